@@ -1,0 +1,596 @@
+"""The work that users of this framework have it do, as cases to measure.
+
+A case is a dict of plain values; its "kind" says which public entry points
+it goes through:
+
+  flow     a simulation from a given state to the next snapshot:
+           Simulation.upload, .run (or .step, one at a time), .state
+  stages   the Particles methods one by one, with their readbacks, as the
+           host classes and analysis programs call them
+  riemann  the batched exact Riemann solver on states in GPU memory
+  train    building the seed network's training set from recorded face
+           problems and training on it (online retraining)
+
+Problems of the flow and stages kinds: "shear" (2D Kelvin-Helmholtz layer on
+a lattice), "shear_random" (the same on random positions), "blast" (3D point
+explosion on a lattice), "turbulence" (3D jittered lattice with a solenoidal
+Mach-1 velocity field), "open" (3D, no periodic boundaries).  The shear
+lattice takes the limiter's intended fabs(): the integer abs() of the default
+turns the 0/0 ratios of its fields, uniform along x up to round-off, into
+-2^31, and the result into amplified round-off.
+"""
+import ctypes as C
+import math
+
+import numpy as np
+import torch
+
+from meshlesshydro_amd import ics, learned, lib, turbulence
+from meshlesshydro_amd._abi import (MLH_ABS_FABS, MLH_ABS_INT_X86, MLH_FP32, MLH_FP64,
+                                    MLH_SEED_LEARNED, MLH_SEED_STANDARD, default_params)
+
+GAMMA = 5.0 / 3.0
+
+
+def flow(name, problem, n, steps, precision, **kw):
+    return dict(kind="flow", name=name, problem=problem, n=n, steps=steps, precision=precision, **kw)
+
+
+def listed():
+    return [
+        # the smallest calls: a first look at a problem, one CFL step per
+        # call; launches and latency count
+        flow("shear 32 fp64 steps", "shear", 32, 4, "fp64", single=True),
+        # the reference's own test problem, 10^4 particles, to a snapshot
+        flow("shear 100 fp64", "shear", 100, 20, "fp64"),
+        # unordered particles of an odd number, the pairwise limiter on
+        flow("shear 181 random fp64", "shear_random", 181, 6, "fp64", pairwise=True),
+        # the million-particle shear layer in the fast precision
+        flow("shear 1000 fp32", "shear", 1000, 10, "fp32"),
+        # the 3D point explosion: the accuracy baseline and the fast mode
+        # with the learned Riemann seed (the headline configuration)
+        flow("blast 128 fp64", "blast", 128, 10, "fp64"),
+        flow("blast 128 fp32 learned", "blast", 128, 25, "fp32", learned=True),
+        # turbulent box: every face strongly nonlinear, ragged rows, the
+        # reference's wide list limits
+        flow("turbulence 160 fp32 learned", "turbulence", 160, 6, "fp32", learned=True),
+        # a free-standing cloud of odd size, its search grid rebuilt from the
+        # particles' limits every step (few steps: its surface expands into
+        # vacuum, which the scheme does not survive for long)
+        flow("open 61 fp32", "open", 61, 3, "fp32"),
+        # method by method with readbacks, FP64 turbulence
+        dict(kind="stages", name="stages 48 fp64", problem="turbulence", n=48, precision="fp64"),
+        # Riemann problems in GPU memory over six decades of density and
+        # nine of pressure, vacuum included
+        dict(kind="riemann", name="riemann 2^24 fp64", n=1 << 24, precision="fp64"),
+        dict(kind="riemann", name="riemann 2^26 fp32 learned", n=1 << 26, precision="fp32", learned=True),
+        # one online retraining of the seed network
+        dict(kind="train", name="train 2^18", n=1 << 18, epochs=2, batch=4096),
+    ]
+
+
+def _log(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    kind = rng.choice(["flow2", "flow3", "flow2", "flow3", "flow3", "stages", "riemann", "train"])
+    prec = rng.choice(["fp64", "fp32"])
+    if kind == "flow2":
+        c = dict(kind="flow", problem=rng.choice(["shear", "shear_random"]), n=_log(rng, 24, 1000),
+                 steps=rng.randint(3, 10), precision=prec)
+        if rng.random() < 0.3:
+            c["pairwise"] = True
+        if rng.random() < 0.2:
+            c["mfm"] = True
+        return c
+    if kind == "flow3":
+        c = dict(kind="flow", problem=rng.choice(["blast", "turbulence", "open"]), n=_log(rng, 12, 140),
+                 steps=rng.randint(2, 6), precision=prec)
+        if c["problem"] == "open":
+            c["steps"] = min(c["steps"], 3)
+        if prec == "fp32" and rng.random() < 0.5:
+            c["learned"] = True
+        return c
+    if kind == "stages":
+        return dict(kind="stages", problem=rng.choice(["shear_random", "turbulence", "open"]),
+                    n=_log(rng, 12, 56), precision=prec)
+    if kind == "riemann":
+        c = dict(kind="riemann", n=_log(rng, 1000, 1 << 25), precision=prec)
+        if rng.random() < 0.5:
+            c["learned"] = True
+        return c
+    return dict(kind="train", n=_log(rng, 1 << 13, 1 << 19), epochs=rng.randint(1, 3),
+                batch=rng.choice([1024, 4096]))
+
+
+# ---- problems -----------------------------------------------------------------
+def _problem(case, seed):
+    """(parameters of default_params, state) of a flow or stages case."""
+    n, rng = case["n"], np.random.default_rng(seed)
+    kw = dict(debug_level=0, precision=MLH_FP32 if case["precision"] == "fp32" else MLH_FP64)
+    if case.get("pairwise"):
+        kw["pairwise_limiter"] = 1
+    if case.get("mfm"):
+        kw["mfm"] = 1
+    if case.get("learned"):
+        kw["riemann_seed"] = MLH_SEED_LEARNED
+    p = case["problem"]
+    if p in ("shear", "shear_random"):
+        st = ics.kelvin_helmholtz(n, regular=p == "shear", seed=seed)
+        # the seeded perturbation's amplitude and phase
+        st["vy"] = 0.01 * rng.uniform(0.5, 2.0) * np.sin(4.0 * np.pi * (st["x"] + rng.uniform()))
+        kw.update(kernel_size=(4.0 if p == "shear" else 3.6) / n)
+        if p == "shear":
+            kw.update(limiter_abs=MLH_ABS_FABS)
+        return kw, st
+    kw.update(dim=3)
+    if p == "blast":
+        st = ics.blast_3d(n, E=rng.uniform(0.5, 2.0))
+        # another lattice site as the centre
+        roll = tuple(int(k) for k in rng.integers(0, n, 3))
+        st["u"] = np.roll(st["u"].reshape(n, n, n), roll, (0, 1, 2)).ravel()
+        kw.update(kernel_size=ics.blast_kernel_size(n), max_interactions=96, max_ghost_interactions=96)
+        return kw, st
+    x, y, z = turbulence.jittered_lattice(n, seed=seed)
+    h, N = turbulence.kernel_size(n), n ** 3
+    X = 2.0 * np.pi * np.stack([x, y, z])
+    v = np.zeros((3, N))
+    for k, a in ((2, 1.0), (3, 0.44), (5, 0.16)):  # divergence-free: component c varies along c + 1 and c + 2
+        ph = rng.uniform(0, 2 * np.pi, (3, 2))
+        for c in range(3):
+            v[c] += a * (np.sin(k * X[(c + 1) % 3] + ph[c, 0]) + np.cos(k * X[(c + 2) % 3] + ph[c, 1]))
+    # rms Mach number at rho = P = 1; the free surface takes a gentler flow
+    v *= (0.3 if p == "open" else 1.0) * math.sqrt(GAMMA) / math.sqrt(np.mean(np.sum(v * v, axis=0)))
+    st = dict(x=x, y=y, z=z, vx=v[0], vy=v[1], vz=v[2], m=np.full(N, 1.0 / N), u=np.full(N, 1.0 / (GAMMA - 1.0)))
+    kw.update(kernel_size=h, max_interactions=400, max_ghost_interactions=300)
+    if p == "open":
+        kw.update(periodic=0)
+    return kw, st
+
+
+def _riemann_states(n, seed, device):
+    """ics.riemann_states' distributions, drawn on `device`: float64 [6, n]."""
+    g = torch.Generator(device=device).manual_seed(seed)
+    r = torch.rand((5, n), generator=g, device=device, dtype=torch.float64)
+    s = torch.zeros((6, n), device=device, dtype=torch.float64)
+    s[0], s[3] = 10.0 ** (6.0 * r[0] - 3.0), 10.0 ** (6.0 * r[1] - 3.0)
+    s[2], s[5] = 10.0 ** (9.0 * r[2] - 6.0), 10.0 ** (9.0 * r[3] - 6.0)
+    cs = 0.5 * (torch.sqrt(GAMMA * s[2] / s[0]) + torch.sqrt(GAMMA * s[5] / s[3]))
+    s[4] = (20.0 * r[4] - 10.0) * cs
+    return s
+
+
+def _faces(n, seed):
+    return np.stack(ics.riemann_states(n, seed=seed), axis=1)
+
+
+def _one_particle():
+    """A handle for the calls that need no particles (weights, stream)."""
+    st = {k: np.array([0.5]) for k in ("x", "y", "m", "u")} | {k: np.zeros(1) for k in ("vx", "vy")}
+    return lib.Simulation(default_params(kernel_size=0.1), st)
+
+
+def _trained(sim, seed):
+    sim.mlp_set_params(learned.init_params(seed))
+    sim.mlp_train_faces(_faces(1 << 14, seed), GAMMA, epochs=2, batch=1024)
+
+
+def prepare(case, seed):
+    kind = case["kind"]
+    if kind in ("flow", "stages"):
+        kw, st = _problem(case, seed)
+        sim = lib.Simulation(default_params(**kw), st)
+        if case.get("learned"):
+            _trained(sim, 1 + seed % 1000)
+        return dict(case=case, sim=sim, initial=st)
+    sim = _one_particle()
+    if kind == "riemann":
+        if case.get("learned"):
+            _trained(sim, 1 + seed % 1000)
+        n = case["n"]
+        return dict(case=case, sim=sim, states=_riemann_states(n, seed, "cuda"),
+                    star=torch.empty((3, n), device="cuda", dtype=torch.float64),
+                    flag=torch.empty(n, device="cuda", dtype=torch.int32))
+    return dict(case=case, sim=sim, faces=_faces(case["n"], seed), weights=learned.init_params(1 + seed % 1000))
+
+
+def run(state):
+    case, sim = state["case"], state["sim"]
+    kind = case["kind"]
+    if kind == "flow":
+        sim.upload(state["initial"])
+        if case.get("single"):
+            dts = np.array([sim.step() for _ in range(case["steps"])])
+        else:
+            dts = sim.run(case["steps"])
+        return {"dt": dts, **sim.state()}
+    if kind == "stages":
+        sim.upload(state["initial"])
+        sim.neighbours()
+        sim.density()
+        rho, P, omega = sim.get_density()
+        dt = sim.timestep()
+        sim.gradients()
+        grads, B = sim.get_gradients()
+        sim.fluxes(dt)
+        mF, vF, eF = sim.get_fluxes()
+        sim.update()
+        return {"rho": rho, "P": P, "omega": omega, "dt": dt, "grads": grads, "B": B, "mF": mF, "vF": vF,
+                "eF": eF, **sim.state()}
+    if kind == "riemann":
+        st, star, flag = state["states"], state["star"], state["flag"]
+        ptr = lambda t: C.c_void_p(t.data_ptr())  # noqa: E731
+        fallbacks, ms = C.c_int64(), (C.c_float * 1)()
+        L = lib.lib()
+        err = L.mlh_riemann_exact_batch_device(
+            sim.h, case["n"], GAMMA, ptr(st), ptr(star), ptr(flag), None,
+            MLH_FP32 if case["precision"] == "fp32" else MLH_FP64,
+            MLH_SEED_LEARNED if case.get("learned") else MLH_SEED_STANDARD, 1e-6, C.byref(fallbacks), ms)
+        if err:
+            raise lib.MLHError(err, "mlh_riemann_exact_batch_device", L.mlh_last_error().decode())
+        return {"star": star, "flag": flag}
+    sim.mlp_set_params(state["weights"])
+    info = sim.mlp_train_faces(state["faces"], GAMMA, epochs=case["epochs"], batch=case["batch"])
+    return {"weights": sim.mlp_get_params(), "train_faces": info["train_faces"], "val_faces": info["val_faces"],
+            "loss": np.array([info["loss_init"], info["loss_final"]], np.float32)}
+
+
+# ---- the work no implementation can do without -----------------------------------
+def _neighbours(case):
+    return {"shear": 45, "shear_random": 41, "blast": 56}.get(case["problem"], 64)
+
+
+def work(case):
+    kind, n = case["kind"], case["n"]
+    if kind == "riemann":
+        # six doubles in, three and a flag out; about 3 Newton iterations of
+        # both sides' pressure functions, guess and sampling
+        return {"bytes": 76.0 * n, "flops": 300.0 * n}
+    if kind == "train":
+        # forward and backward of 10-64-64-1 per sample and epoch, p* per face
+        return {"bytes": 48.0 * n, "flops": n * (case["epochs"] * 6.0 * (10 * 64 + 64 * 64 + 64) + 1000.0)}
+    D = 2 if case["problem"].startswith("shear") else 3
+    N, k = n ** D, _neighbours(case)
+    # per step: the state in and out; per undirected pair the distance and
+    # kernel (20), E, gradients and extrema (60), the limiter (30), both
+    # face states, the Riemann problem and the flux (250), all sums
+    steps = case.get("steps", 1)
+    state = 8.0 * (2 * D + 2)
+    extra = 8.0 * ((D + 2) * D + D * D + 3 + D + 2) if kind == "stages" else 0.0
+    return {"bytes": N * (steps * 2 * state + extra), "flops": N * steps * (0.5 * k * 360.0)}
+
+
+# ---- the same results in 64 bits, plain torch -------------------------------------
+# directed pairs times steps beyond which the values are not computed here
+EXACT_MOST = 1.2e9
+
+
+def exact(case, seed):
+    dev = "cuda" if torch.cuda.is_available() else "cpu"
+    kind = case["kind"]
+    if kind == "riemann":
+        s = _riemann_states(case["n"], seed, dev)
+        if case["precision"] == "fp32":
+            s = s.float().double()
+        out = torch.empty((3, case["n"]), dtype=torch.float64, device=dev)
+        for a in range(0, case["n"], 1 << 22):
+            out[:, a:a + (1 << 22)] = torch.stack(_riemann(*s[:, a:a + (1 << 22)])[:3])
+        return {"star": out, "flag": None}
+    if kind == "train":
+        w, loss = _train64(case, _faces(case["n"], seed), learned_init(1 + seed % 1000), dev)
+        return {"weights": w, "train_faces": None, "val_faces": None, "loss": loss}
+    N = case["n"] ** (2 if case["problem"].startswith("shear") else 3)
+    if N * _neighbours(case) * case.get("steps", 1) > EXACT_MOST:
+        return None
+    kw, st = _problem(case, seed)
+    D = kw.get("dim", 2)
+    t = lambda k: torch.as_tensor(st[k], dtype=torch.float64, device=dev)  # noqa: E731
+    x = torch.stack([t(k) for k in "xyz"[:D]], 1)
+    v = torch.stack([t(k) for k in ("vx", "vy", "vz")[:D]], 1)
+    m, u = t("m"), t("u")
+    dts = []
+    for _ in range(case.get("steps", 1)):
+        x, v, m, u, dt, mid = _step64(kw, x, v, m, u)
+        dts.append(dt)
+    out = {k: x[:, a].contiguous() for a, k in enumerate("xyz"[:D])}
+    out |= {k: v[:, a].contiguous() for a, k in enumerate(("vx", "vy", "vz")[:D])}
+    out |= {"m": m, "u": u}
+    if kind == "flow":
+        return {"dt": np.array(dts), **out}
+    return {**mid, "dt": dts[0], **out}
+
+
+def learned_init(seed):
+    """Glorot-uniform hidden layers, zero biases and output layer."""
+    rng, p, H = np.random.default_rng(seed), np.zeros(4929, np.float32), 64
+    a, b = math.sqrt(6.0 / (10 + H)), math.sqrt(6.0 / (H + H))
+    p[:640] = rng.uniform(-a, a, 640)
+    p[704:704 + 4096] = rng.uniform(-b, b, 4096)
+    return p
+
+
+def _riemann(dl, ul, pl, dr, ur, pr):
+    """Exact solution at x/t = 0 (gamma = 5/3): rho, u, p and the upwind side."""
+    g = GAMMA
+    cl, cr, du = torch.sqrt(g * pl / dl), torch.sqrt(g * pr / dr), ur - ul
+    vac = 2 / (g - 1) * (cl + cr) <= du
+
+    def f(p, d, pk, c):
+        q = torch.sqrt(2 / (g + 1) / d / ((g - 1) / (g + 1) * pk + p))
+        r = (p / pk) ** ((g - 1) / (2 * g))
+        rare = p <= pk
+        return (torch.where(rare, 2 / (g - 1) * c * (r - 1), (p - pk) * q),
+                torch.where(rare, r / (p / pk) / (d * c), (1 - 0.5 * (p - pk) / (p + (g - 1) / (g + 1) * pk)) * q))
+
+    # two rarefactions: below the root (f is increasing and concave), from
+    # where Newton's method rises to it
+    e = (g - 1) / (2 * g)
+    num = (cl + cr - 0.5 * (g - 1) * du).clamp_min(0)
+    tiny = 1e-14 * torch.minimum(pl, pr)
+    p = torch.maximum((num / (cl / pl ** e + cr / pr ** e)) ** (1 / e), tiny)
+    for _ in range(60):
+        fl, gl = f(p, dl, pl, cl)
+        fr, gr = f(p, dr, pr, cr)
+        q = torch.maximum(p - (fl + fr + du) / (gl + gr), tiny)
+        done = bool((((q - p).abs() <= 1e-15 * (q + p)) | vac).all())
+        p = q
+        if done:
+            break
+    fl, fr = f(p, dl, pl, cl)[0], f(p, dr, pr, cr)[0]
+    us = 0.5 * (ul + ur + fr - fl)
+    # sample: mirror the right side's problem onto the left's
+    left = us >= 0
+    s = torch.where(left, 1.0, -1.0)
+    pk, c = torch.where(left, pl, pr), torch.where(left, cl, cr)
+    d = torch.where(left, dl, dr)
+    u = s * torch.where(left, ul, ur)
+    um, P = s * us, p / pk
+    G = (g - 1) / (g + 1)
+    shock = p > pk
+    outside = torch.where(shock, u - c * torch.sqrt((g + 1) / (2 * g) * P + e), u - c) >= 0
+    cc = (2 / (g + 1) + G / c * u).clamp_min(0)  # in the fan: c* / c
+    fan = ~shock & (um - c * P ** e > 0)
+    ro = torch.where(shock, d * (P + G) / (G * P + 1), torch.where(fan, d * cc ** (2 / (g - 1)), d * P ** (1 / g)))
+    uo = torch.where(fan, 2 / (g + 1) * (c + 0.5 * (g - 1) * u), um)
+    po = torch.where(fan, pk * cc ** (2 * g / (g - 1)), p)
+    ro, uo, po = torch.where(outside, d, ro), s * torch.where(outside, u, uo), torch.where(outside, pk, po)
+    side = torch.where(left, -1, 1)
+    if bool(vac.any()):
+        # vacuum opens between the two rarefactions
+        shl, stl, shr, strr = ul - cl, ul + 2 / (g - 1) * cl, ur + cr, ur - 2 / (g - 1) * cr
+        z = torch.zeros_like(dl)
+        a, b = (2 / (g + 1) + G / cl * ul).clamp_min(0), (2 / (g + 1) - G / cr * ur).clamp_min(0)
+        vals = [(shl >= 0, dl, ul, pl, -1), (stl > 0, dl * a ** (2 / (g - 1)), 2 / (g + 1) * (cl + 0.5 * (g - 1) * ul), pl * a ** (2 * g / (g - 1)), -1),
+                (shr <= 0, dr, ur, pr, 1), (strr < 0, dr * b ** (2 / (g - 1)), 2 / (g + 1) * (-cr + 0.5 * (g - 1) * ur), pr * b ** (2 * g / (g - 1)), 1)]
+        R, U, Q, S = z, z, z, torch.zeros_like(side)
+        for cond, rr, uu, pp, ss in reversed(vals):
+            R, U, Q, S = torch.where(cond, rr, R), torch.where(cond, uu, U), torch.where(cond, pp, Q), torch.where(cond, ss, S)
+        ro, uo, po, side = torch.where(vac, R, ro), torch.where(vac, U, uo), torch.where(vac, Q, po), torch.where(vac, S, side)
+    return ro, uo, po, side, p
+
+
+def _pairs(kw, x):
+    """All directed pairs within h: i, j, x_j - x_i, whether j is an image."""
+    N, D = x.shape
+    h, per = kw["kernel_size"], kw.get("periodic", 1)
+    lo = torch.zeros(D, dtype=x.dtype, device=x.device) if per else x.amin(0)
+    ext = torch.ones_like(lo) if per else x.amax(0) - lo
+    nc = [max(1, int(e / h * (1 - 1e-12))) for e in ext.tolist()]
+    cell = torch.stack([((x[:, a] - lo[a]) / ext[a] * nc[a]).long().clamp(0, nc[a] - 1) for a in range(D)], 1)
+
+    def key(c):
+        k = c[:, 0]
+        for a in range(1, D):
+            k = k * nc[a] + c[:, a]
+        return k
+
+    ks, order = torch.sort(key(cell))
+    out = []
+    for o in range(3 ** D):
+        off = torch.tensor([(o // 3 ** a) % 3 - 1 for a in range(D)], device=x.device)
+        c = cell + off
+        shift = torch.zeros_like(x)
+        ok = torch.ones(N, dtype=torch.bool, device=x.device)
+        for a in range(D):
+            low, high = c[:, a] < 0, c[:, a] >= nc[a]
+            if per:
+                shift[:, a] = high.double() - low.double()
+                c[:, a] = c[:, a] + nc[a] * (low.long() - high.long())
+            else:
+                ok &= ~low & ~high
+        k = torch.where(ok, key(c), -1)
+        s, e = torch.searchsorted(ks, k), torch.searchsorted(ks, k, right=True)
+        cnt = torch.where(ok, e - s, 0)
+        i = torch.repeat_interleave(torch.arange(N, device=x.device), cnt)
+        j = order[s[i] + torch.arange(len(i), device=x.device) - (cnt.cumsum(0) - cnt)[i]]
+        d = x[j] + shift[i] - x[i]
+        img = (shift[i] != 0).any(1)
+        keep = ((d * d).sum(1) < h * h) & ((i != j) | img)
+        out.append((i[keep], j[keep], d[keep], img[keep]))
+    return [torch.cat(t) for t in zip(*out)]
+
+
+def _w(r, h, D):
+    h2 = h / 2
+    sig = 10 / (7 * math.pi * h2 ** 2) if D == 2 else 1 / (math.pi * h2 ** 3)
+    q = r / h2
+    return sig * torch.where(q <= 1, 1 - 1.5 * q * q * (1 - q / 2), 0.25 * (2 - q).clamp_min(0) ** 3)
+
+
+def _abs(a, mode):
+    """The limiters' abs(): |a|, or abs() of the value as a 32-bit integer."""
+    if mode == MLH_ABS_FABS:
+        return a.abs()
+    bad = ~(a.abs() < 2147483648.0)
+    return torch.where(bad, -2147483648.0, torch.where(bad, 0.0, a).trunc().abs())
+
+
+def _pairwise(phi0, fi, fj, part, mode):
+    bar, diff = fi + part * (fj - fi), _abs(fi - fj, mode)
+    d1, d2, lo, hi = 0.5 * diff, 0.25 * diff, torch.minimum(fi, fj), torch.maximum(fi, fj)
+    up = torch.where(((hi + d1) >= 0) == (hi >= 0), hi + d1, hi / (1 + d1 / _abs(hi, mode)))
+    dn = torch.where(((lo - d1) >= 0) == (lo >= 0), lo - d1, lo / (1 + d1 / _abs(lo, mode)))
+    return torch.where(fi < fj, torch.maximum(dn, torch.minimum(bar + d2, phi0)),
+                       torch.where(fi > fj, torch.minimum(up, torch.maximum(bar - d2, phi0)), fi))
+
+
+def _step64(kw, x, v, m, u):
+    """One step of the meshless finite volume scheme, every directed face from its own particle."""
+    N, D = x.shape
+    h, mode = kw["kernel_size"], kw.get("limiter_abs", MLH_ABS_INT_X86)
+    i, j, d, img = _pairs(kw, x)
+    sums = lambda t: torch.zeros((N,) + t.shape[1:], dtype=t.dtype, device=t.device).index_add_(0, i, t)  # noqa: E731
+
+    def ext(t, start, how):
+        o = torch.full((N,) + t.shape[1:], start, dtype=t.dtype, device=t.device)
+        ix = i if t.dim() == 1 else i[:, None].expand_as(t)
+        return o.scatter_reduce_(0, ix, t, how)
+
+    r = torch.sqrt((d * d).sum(1))
+    w = _w(r, h, D)
+    om = sums(w) + float(_w(torch.zeros(1, dtype=torch.float64), h, D))
+    rho = m * om
+    P = (GAMMA - 1) * rho * u
+    c = torch.sqrt(GAMMA * P / rho)
+    f = torch.cat([rho[:, None], v, P[:, None]], 1)
+    vx = -((v[i] - v[j]) * d).sum(1) / r
+    vsig = ext(torch.where(img, 2.3e-308, c[i] + c[j] - vx.clamp_max(0)), 2.3e-308, "amax")
+    dt = float((0.4 * h / vsig).min())
+    wi = (w / om[i])[:, None]
+    B = torch.linalg.inv(sums((d[:, :, None] * d[:, None, :]).reshape(-1, D * D) * wi).reshape(N, D, D))
+    # grad f = B sum (f_j - f_i) (x_j - x_i) W / omega
+    G = torch.stack([(B @ sums((f[j, k] - f[i, k])[:, None] * d * wi)[:, :, None])[:, :, 0] for k in range(D + 2)], 1)
+    for k in range(D + 2):
+        hi, lo = ext(f[j, k], 2.3e-308, "amax"), ext(f[j, k], 1.7e308, "amin")
+        dj = 0.5 * (G[i, k] * d).sum(1)
+        mhi = (f[:, k] + ext(dj, -math.inf, "amax")).clamp_min(2.3e-308)
+        mlo = (f[:, k] + ext(dj, math.inf, "amin")).clamp_max(1.7e308)
+        amax, amin = _abs((hi - f[:, k]) / (mhi - f[:, k]), mode), _abs((f[:, k] - lo) / (f[:, k] - mlo), mode)
+        fac = torch.where((amin <= amax) & (4 * amin < 1), amin, torch.where((amax <= amin) & (4 * amax < 1), amax, 1.0))
+        G[:, k] = G[:, k] * fac[:, None]
+    F = torch.zeros((N, D + 2), dtype=x.dtype, device=x.device)
+    for a in range(0, len(i), 1 << 23):
+        q = slice(a, a + (1 << 23))
+        F.index_add_(0, i[q], _faces64(kw, D, i[q], j[q], d[q], img[q], r[q], w[q], om, B, f, G, dt))
+    m1 = m if kw.get("mfm") else m - dt * F[:, 0]
+    vn = (m[:, None] * v - dt * F[:, 2:]) / m1[:, None]
+    un = (m * (u + 0.5 * (v * v).sum(1)) - dt * F[:, 1]) / m1 - 0.5 * (vn * vn).sum(1)
+    xn = x + v * dt
+    if kw.get("periodic", 1):
+        xn = torch.where(xn < 0, xn + 1, torch.where(xn >= 1, xn - 1, xn))
+    mid = {"rho": rho, "P": P, "omega": om, "grads": G.permute(1, 0, 2).contiguous(), "B": B,
+           "mF": F[:, 0].contiguous(), "eF": F[:, 1].contiguous(), "vF": F[:, 2:].contiguous()}
+    return xn, vn, m1, un, dt, mid
+
+
+def _faces64(kw, D, i, j, d, img, r, w, om, B, f, G, dt):
+    """Fluxes (mass, energy, momentum) through the faces of pairs i, j as seen from i."""
+    A = ((B[i] @ d[:, :, None])[:, :, 0] * (w / om[i] ** 2)[:, None] + (B[j] @ d[:, :, None])[:, :, 0] * (w / om[j] ** 2)[:, None])
+    vF = 0.5 * (f[i, 1:D + 1] + f[j, 1:D + 1])
+
+    def side(k, sgn):
+        W = f[k].clone()
+        W[:, 1:D + 1] -= vF
+        return W, W + sgn * 0.5 * (G[k] * d[:, None, :]).sum(2)
+
+    bi, Wi = side(i, 1.0)
+    bj, Wj = side(j, -1.0)
+    if kw.get("pairwise_limiter"):
+        mode = kw.get("limiter_abs", MLH_ABS_INT_X86)
+        Li, Lj = (torch.stack([_pairwise(W[:, k], p[:, k], q[:, k], 0.5, mode) for k in range(D + 2)], 1)
+                  for W, p, q in ((Wi, bi, bj), (Wj, bj, bi)))
+        Wi, Wj = torch.where(img[:, None], Wi, Li), torch.where(img[:, None], Wj, Lj)
+
+    def half(W, b, k):
+        g, vr = G[k], b[:, 1:D + 1]
+        div = sum(g[:, 1 + a, a] for a in range(D))
+        W = W.clone()
+        W[:, 0] -= dt / 2 * (b[:, 0] * div + (vr * g[:, 0]).sum(1))
+        W[:, D + 1] -= dt / 2 * (GAMMA * b[:, D + 1] * div + (vr * g[:, D + 1]).sum(1))
+        for a in range(D):
+            W[:, 1 + a] -= dt / 2 * (g[:, D + 1, a] / b[:, 0] + (vr * g[:, 1 + a]).sum(1))
+        return W
+
+    Wi, Wj = half(Wi, bi, i), half(Wj, bj, j)
+    An = torch.sqrt((A * A).sum(1))
+    some = An > 0
+    n = A / torch.where(some, An, 1.0)[:, None]
+    ui, uj = (n * Wi[:, 1:D + 1]).sum(1), (n * Wj[:, 1:D + 1]).sum(1)
+    rs, us, Ps, side_, _ = _riemann(Wi[:, 0], ui, Wi[:, D + 1], Wj[:, 0], uj, Wj[:, D + 1])
+    up = torch.where((side_ == 1)[:, None], Wj[:, 1:D + 1] - uj[:, None] * n, Wi[:, 1:D + 1] - ui[:, None] * n)
+    vS = us[:, None] * n + torch.where((side_ == 0)[:, None], 0.0, up)
+    lab = vS + vF
+    Av = (A * vS).sum(1)
+    mass = rs * Av
+    adv = torch.zeros_like(Av) if kw.get("mfm") else Av
+    en = adv * (Ps / (GAMMA - 1) + 0.5 * rs * (lab * lab).sum(1)) + Ps * (A * lab).sum(1)
+    mom = (adv * rs)[:, None] * lab + Ps[:, None] * A
+    return torch.where(some[:, None], torch.cat([mass[:, None], en[:, None], mom], 1), 0.0)
+
+
+def _mix64(z):
+    with np.errstate(over="ignore"):
+        z = np.asarray(z, np.uint64) + np.uint64(0x9E3779B97F4A7C15)
+        z = (z ^ (z >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
+        z = (z ^ (z >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
+        return z ^ (z >> np.uint64(31))
+
+
+def _train64(case, faces, w0, dev):
+    """The training set's rules (the header of mlh_mlp_train_faces) and Adam in 64 bits: weights, (first, last) loss."""
+    g = GAMMA
+    dl, ul, pl, dr, ur, pr = (torch.as_tensor(faces[:, k], dtype=torch.float64, device=dev) for k in range(6))
+    cl, cr, du, pref = torch.sqrt(g * pl / dl), torch.sqrt(g * pr / dr), ur - ul, 0.5 * (pl + pr)
+    ps = torch.where(2 / (g - 1) * (cl + cr) <= du, 0.0, _riemann(dl, ul, pl, dr, ur, pr)[4])
+    ppv = (pref - 0.125 * du * (dl + dr) * (cl + cr)).clamp_min(0)
+    e = (g - 1) / (2 * g)
+    pq = (pl / pr) ** e
+    um = (pq * ul / cl + ur / cr + 2 / (g - 1) * (pq - 1)) / (pq / cl + 1 / cr)
+    tl, tr = 1 + 0.5 * (g - 1) * (ul - um) / cl, 1 + 0.5 * (g - 1) * (um - ur) / cr
+    trr = torch.where((tl > 0) & (tr > 0), 0.5 * (pl * tl.clamp_min(0) ** (1 / e) + pr * tr.clamp_min(0) ** (1 / e)), 0.0)
+    G, p0 = (g - 1) / (g + 1), torch.maximum(ppv, 1e-6 * pref)
+    gl, gr = torch.sqrt(2 / (g + 1) / dl / (G * pl + p0)), torch.sqrt(2 / (g + 1) / dr / (G * pr + p0))
+    tss = (gl * pl + gr * pr - du) / (gl + gr)
+    pmin, pmax = torch.minimum(pl, pr), torch.maximum(pl, pr)
+    pg = torch.where((pmax / pmin <= 2) & (pmin <= ppv) & (ppv <= pmax), ppv, torch.where(ppv < pmin, trr, tss))
+    lg = lambda t: torch.log(t.clamp_min(1e-30)).clamp(-40, 5)  # noqa: E731
+    X = torch.stack([lg(pl / pref), lg(pr / pref), du / (cl + cr), (cl - cr) / (cl + cr), lg(ppv / pref), lg(trr / pref),
+                     lg(tss / pref), lg(pg / pref), torch.full_like(dl, G), lg(dl / dr) / 4], 1)
+    T = torch.log(ps.clamp_min(1e-300) / pref) - X[:, 7]
+    hk = np.zeros(len(faces), np.uint64)
+    bits = np.ascontiguousarray(faces).view(np.uint64)
+    for k in range(6):
+        hk = _mix64(hk ^ bits[:, k])
+    ok, trivial = (ps > 0).cpu().numpy(), (T.abs() < 1e-5).cpu().numpy()
+    nt, ntr = int((ok & ~trivial).sum()), int((ok & trivial).sum())
+    keep = min(ntr, max(max(nt, 1), 1024))
+    thr = 0 if ntr == 0 else 1 << 53 if keep >= ntr else int(keep / ntr * 9007199254740992.0)
+    sel = np.flatnonzero(ok & (~trivial | ((_mix64(hk ^ np.uint64(0x5851F42D4C957F2D)) >> np.uint64(11)) < np.uint64(thr))))
+    hs = hk[sel]
+    sel = torch.as_tensor(sel[np.lexsort((hs & np.uint64(0xFFFFFFFF), hs >> np.uint64(33)))], device=dev)
+    X, T = X[sel], T[sel]
+    n = len(T)
+    nval = max(n // 10, 64)
+    batch = min(case["batch"], n - nval)
+    w = torch.as_tensor(w0, dtype=torch.float64, device=dev).requires_grad_()
+
+    def loss(a, b):
+        h = torch.tanh(a @ w[:640].view(64, 10).T + w[640:704])
+        h = torch.tanh(h @ w[704:4800].view(64, 64).T + w[4800:4864])
+        return ((h @ w[4864:4928] + w[4928] - b) ** 2).mean()
+
+    first, last, t = float(loss(X[:65536], T[:65536])), 0.0, 0
+    M, V = torch.zeros_like(w), torch.zeros_like(w)
+    with np.errstate(over="ignore"):
+        base = _mix64(np.uint64(1) ^ np.uint64(0xA0761D6478BD642F))
+        for ep in range(case["epochs"]):
+            key = _mix64(_mix64(base + np.uint64(ep)) ^ np.arange(n - nval, dtype=np.uint64)) >> np.uint64(32)
+            order = torch.as_tensor(nval + np.argsort(key, kind="stable"), device=dev)
+            for a in range(0, n - nval - batch + 1, batch):
+                L = loss(X[order[a:a + batch]], T[order[a:a + batch]])
+                gr_, = torch.autograd.grad(L, w)
+                t, last = t + 1, float(L)
+                M, V = 0.9 * M + 0.1 * gr_, 0.999 * V + 0.001 * gr_ * gr_
+                w = (w - 2e-3 * (M / (1 - 0.9 ** t)) / (torch.sqrt(V / (1 - 0.999 ** t)) + 1e-8)).detach().requires_grad_()
+    return w.detach(), np.array([first, last])
