@@ -173,7 +173,7 @@ def _one_particle():
 
 def _trained(sim, seed):
     sim.mlp_set_params(learned.init_params(seed))
-    sim.mlp_train_faces(_faces(1 << 14, seed), GAMMA, epochs=2, batch=1024)
+    sim.mlp_train_faces(_faces(1 << 18, seed), GAMMA, epochs=4, batch=4096)
 
 
 def prepare(case, seed):
