@@ -51,6 +51,14 @@ struct mlh_ctx {
     int cell_cap = 0;                // cells cstart / cend can hold
     double *lim_scratch = nullptr;   // domain limits (non-periodic)
     double *lim_out = nullptr;
+    // the faces' fluxes, evaluated once per pair (HydroArgs::flux): own
+    // allocation, grown between calls when the lists need more slots
+    void *flux = nullptr;
+    unsigned long long flux_cap = 0;
+    bool flux_fits = false;
+    uint16_t *face_rec = nullptr;
+    uint2 *deferred = nullptr;  // (re)allocated with flux
+    unsigned long long *nfaces = nullptr;
     uint32_t *nbr = nullptr;
     int *noi = nullptr, *nog = nullptr;
     void *prim = nullptr, *frec = nullptr;
@@ -185,6 +193,58 @@ static int make_geom(mlh_ctx *c, const double *lo, const double *hi) {
     return 0;
 }
 
+// Slots for the faces' fluxes.  Without memory for them (or with rows too
+// long for the records) every face is evaluated from both sides.
+constexpr size_t kFluxSmall = 64u << 20;   // bytes: given for the longest lists
+constexpr int kFluxPerParticle = 40;       // else at first: half of 72
+                                           // neighbours, and some images
+static void set_flux_slots(mlh_ctx *c, unsigned long long cap) {
+    const size_t bytes = (size_t)(c->D + 2) * c->tsz;
+    if (cap > 0xfffffff0ull) cap = 0xfffffff0ull;
+    void *q = nullptr;
+    uint2 *d = nullptr;
+    // FP32 learned: the list of rounds with deferred faces: 64 faces each but
+    // the last two of a group (of four particles at least)
+    if (c->prec == MLH_FP32 && c->p.riemann_seed == MLH_SEED_LEARNED) {
+        const size_t n = 1 + (size_t)cap / 64 + 2 * ((size_t)c->N / 4 + 1);
+        if (hipMalloc((void **)&d, sizeof(uint2) * n) != hipSuccess ||
+            hipMemsetAsync(d, 0, sizeof(uint2), c->s) != hipSuccess) {
+            if (d) hipFree(d);
+            hipGetLastError();
+            return;  // as it was
+        }
+    }
+    if (hipMalloc(&q, bytes * cap) != hipSuccess) {
+        if (d) hipFree(d);
+        hipGetLastError();
+        return;
+    }
+    if (c->flux) hipFree(c->flux);
+    if (c->deferred) hipFree(c->deferred);
+    c->flux = q;
+    c->deferred = d;
+    c->flux_cap = cap;
+}
+static void first_flux_slots(mlh_ctx *c) {
+    const mlh_params &p = c->p;
+    if (p.max_interactions > kFaceRecMaxRow || p.max_ghost_interactions > kFaceRecMaxRow) return;
+    // a real pair has one slot, an image entry its own
+    const unsigned long long N = c->N, D2 = c->D + 2;
+    const unsigned long long rows = p.enforce_flux_sym ? (N * p.max_interactions + 1) / 2
+                                                       : N * p.max_interactions;
+    const unsigned long long all = rows + N * (p.periodic ? p.max_ghost_interactions : 0);
+    c->flux_fits = all * D2 * c->tsz <= kFluxSmall;
+    const unsigned long long some = N * kFluxPerParticle * (p.enforce_flux_sym ? 1 : 2);
+    set_flux_slots(c, c->flux_fits || all < some ? all : some);
+    c->flux_fits = c->flux != nullptr && c->flux_cap >= all;
+}
+// after a call whose faces did not fit (they were evaluated from both sides):
+// room for them and a quarter more
+static void grow_flux_slots(mlh_ctx *c, unsigned long long nfaces) {
+    if (c->flux && nfaces > c->flux_cap && c->flux_cap < 0xfffffff0ull)
+        set_flux_slots(c, nfaces + nfaces / 4);
+}
+
 static HydroArgs hydro_args(mlh_ctx *c) {
     HydroArgs a{};
     const mlh_params &p = c->p;
@@ -211,6 +271,14 @@ static HydroArgs hydro_args(mlh_ctx *c) {
     a.nbr = c->nbr;
     a.noi = c->noi;
     a.nog = c->nog;
+    a.flux = c->flux;
+    a.face_rec = c->face_rec;
+    a.deferred = c->deferred;
+    a.nfaces = c->nfaces;
+    a.fcap = c->flux_cap;
+    a.flux_fits = c->flux_fits ? 1 : 0;
+    a.maxr = p.max_interactions;
+    a.ck = co ? c->cell_key : c->sorted_key;
     for (int k = 0; k < 3; ++k) {
         a.x[k] = c->x[k]; a.v[k] = c->v[k];
         a.xn[k] = c->xn[k]; a.vn[k] = c->vn[k];
@@ -305,13 +373,17 @@ int mlh_create(const mlh_params *p, int32_t n, mlh_ctx **out) {
     A_(&c->dt, sizeof(double) * 4);
     A_(&c->mF, dsz); A_(&c->vF, dsz * D); A_(&c->eF, dsz);
     A_(&c->counters, sizeof(unsigned long long) * kNumCounters);
-    A_(&c->status, sizeof(int) * 2);
+    // status words, then the face-slot counter (read back together)
+    A_(&c->status, sizeof(int) * 2 + sizeof(unsigned long long));
+    c->nfaces = (unsigned long long *)(c->status + 2);
+    A_(&c->face_rec, sizeof(uint16_t) * (D == 2 ? FaceRec<2>::N : FaceRec<3>::N) * N);
     A_(&c->max_counts, sizeof(int) * 2);
     A_(&c->sums_block, sizeof(double) * 6 * (size_t)dt_blocks(n));
 #undef A_
     hipMemsetAsync(c->counters, 0, sizeof(unsigned long long) * kNumCounters, c->s);
     hipMemsetAsync(c->status, 0, sizeof(int), c->s);
     hipMemsetAsync(c->status + 1, 0xff, sizeof(int), c->s);
+    hipMemsetAsync(c->nfaces, 0, sizeof(unsigned long long), c->s);
     hipMemsetAsync(c->max_counts, 0, sizeof(int) * 2, c->s);
     hipMemsetAsync(c->noi, 0, 4 * N, c->s);
     hipMemsetAsync(c->nog, 0, 4 * N, c->s);
@@ -324,6 +396,7 @@ int mlh_create(const mlh_params *p, int32_t n, mlh_ctx **out) {
         mlh_destroy(c);
         return fail(MLH_ERR_DEVICE, "initialisation failed");
     }
+    first_flux_slots(c);
     *out = c;
     return MLH_OK;
 }
@@ -339,6 +412,8 @@ int mlh_destroy(mlh_ctx *c) {
     mlp_free(c->mlp);
     for (hipEvent_t e : c->evpool) hipEventDestroy(e);
     if (c->dt_hist) hipFree(c->dt_hist);
+    if (c->flux) hipFree(c->flux);
+    if (c->deferred) hipFree(c->deferred);
     if (c->s_img) hipStreamSynchronize(c->s_img);
     if (c->ev_fork) hipEventDestroy(c->ev_fork);
     if (c->ev_join) hipEventDestroy(c->ev_join);
@@ -427,7 +502,7 @@ static int enqueue_neighbours(mlh_ctx *c, bool fuse_density = false) {
     }
     launch_cells(c->g, c->D, c->x[0], c->x[1], c->D == 3 ? c->x[2] : c->x[0], c->N, c->pos,
                  c->cell_key, c->sorted_idx, c->sorted_key, c->sort_scratch, c->cstart, c->cend,
-                 c->inv_idx, c->s);
+                 c->inv_idx, c->nfaces, c->s);
     if (c->order == 0) resolve_order(c);
     const bool co = c->order == MLH_ORDER_CALLER;
     if (co)
@@ -453,6 +528,9 @@ static int enqueue_neighbours(mlh_ctx *c, bool fuse_density = false) {
     a.img_window = c->img_window;
     a.img_cnt = c->img_cnt;
     a.img_base = c->img_base;
+    a.face_rec = c->face_rec;
+    a.nfaces = c->nfaces;
+    a.all_own = c->p.enforce_flux_sym ? 0 : 1;
     a.dens = fuse_density ? (c->prec == MLH_FP32 ? 4 : 8) : 0;
     if (fuse_density) {
         a.prim = c->prim;
@@ -491,10 +569,12 @@ static int clear_status(mlh_ctx *c) {
 }
 
 static int check_status(mlh_ctx *c) {
-    int st[2];
-    HIPCHK(hipMemcpyAsync(st, c->status, sizeof(st), hipMemcpyDeviceToHost, c->s));
+    struct { int st[2]; unsigned long long nfaces; } w;
+    HIPCHK(hipMemcpyAsync(&w, c->status, sizeof(w), hipMemcpyDeviceToHost, c->s));
     HIPCHK(hipStreamSynchronize(c->s));
     HIPCHK(hipGetLastError());
+    const int *st = w.st;
+    grow_flux_slots(c, w.nfaces);
     // a run names the step (the state is the one at its start: the face
     // kernel of that step and of every later one keeps the state unchanged)
     const std::string at =

@@ -50,8 +50,10 @@ template <int D>
 __global__ void k_assign_cells(Geom g, const double *__restrict__ x0,
                                const double *__restrict__ x1,
                                const double *__restrict__ x2, int N,
-                               uint32_t *__restrict__ key, uint32_t *__restrict__ idx) {
+                               uint32_t *__restrict__ key, uint32_t *__restrict__ idx,
+                               unsigned long long *__restrict__ nfaces) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) *nfaces = 0;  // the search's face slots
     if (i >= N) return;
     double xs[3] = {x0[i], x1[i], D == 3 ? x2[i] : 0.0};
     int f[3] = {0, 0, 0};
@@ -501,10 +503,13 @@ __device__ inline int image_search(const NbrArgs &a, int t, const double *xi, co
 //    every eight hits are stored as one 32-byte sector of the chunked row.
 //  * The capacity is checked per group of four: the list has four guard
 //    entries past its last one for the overshoot.
-// Returns the real count through cnt_out.
+// Returns the real count through cnt_out, the particle's own faces (those
+// whose slots are handed out here: none yet for a particle with images)
+// through own_out, and its face-slot record in segs (LDS) but for the slot.
 template <int D, bool kCaller, int kDens, typename Src>
 __device__ inline void search_one(const NbrArgs &a, int t, const Src &src, uint32_t *stage,
-                                  int &cnt_out) {
+                                  uint16_t *segs, int &cnt_out, int &own_out) {
+    constexpr int C = FaceRec<D>::C;
     using TW = typename std::conditional<kDens == 4, float, double>::type;
     const Geom &g = a.g;
     const int N = a.N;
@@ -517,7 +522,7 @@ __device__ inline void search_one(const NbrArgs &a, int t, const Src &src, uint3
     uint32_t ck = a.ck_w[t];
     int cc[3];
     cell_coords<D>(g, ck, cc);
-    int err = 0;
+    int err = 0, nb = 0;
     // hits go to the thread's LDS stage (two chunks of eight entries, entry
     // n at stage[n & 15]); each completed chunk is stored as one 32-byte
     // sector of the row, so every sector is written once and whole
@@ -543,6 +548,11 @@ __device__ inline void search_one(const NbrArgs &a, int t, const Src &src, uint3
                 uint32_t c = cell_key<D>(g, k, l, m);
                 int q0, q1, delta;
                 src.range(k, l, m, c, q0, q1, delta);
+                const int sp = D == 2 ? 3 * (k - cc[0]) + (l - cc[1])
+                                      : 9 * (k - cc[0]) + 3 * (l - cc[1]) + (m - cc[2]);
+                const bool own_cell = sp == 0;
+                if (own_cell) nb = cnt;
+                if (sp > 0) segs[2 + sp] = (uint16_t)cnt;
                 for (int q = q0; q < q1; q += 4) {
                     double4 pj[4];
 #pragma unroll
@@ -552,19 +562,22 @@ __device__ inline void search_one(const NbrArgs &a, int t, const Src &src, uint3
                         const int qq = q + u;
                         double xj[3] = {pj[u].x, pj[u].y, pj[u].z};
                         double d = dist2<D>(xj, xi);
-                        bool other;
+                        bool other, before;
                         uint32_t val;
                         if constexpr (kCaller) {
                             const uint32_t jo = (uint32_t)pj[u].w;
                             other = jo != io;
+                            before = jo < io;
                             val = jo;
                         } else {
                             other = qq != t;
+                            before = qq < t;
                             val = (uint32_t)qq;
                         }
                         if (qq < q1 && other && d < g.hsq) {
                             stage[cnt & 15] = val | (kCodeReal << kIdxBits);
                             ++cnt;
+                            if (own_cell && before) ++nb;
                             // density: the hits in row order, with the
                             // distance of the test ((-a)^2 = a^2 exactly)
                             if constexpr (kDens != 0)
@@ -594,6 +607,8 @@ __device__ inline void search_one(const NbrArgs &a, int t, const Src &src, uint3
     // marks it); the others have none
     const bool images = !err && has_images<D>(a, cc);
     a.nog[t] = images ? -1 : 0;
+    segs[2] = (uint16_t)nb;
+    own_out = images ? 0 : (a.all_own ? cnt : (cnt > nb ? cnt - nb : 0));
     if constexpr (kDens != 0) {
         // compDensity (Particles.cpp:1151-1184): the self term after the
         // real neighbours, then the images in ghost order (:2262-2290), which
@@ -623,6 +638,30 @@ __device__ inline void reduce_max_counts(const NbrArgs &a, int cnt, int gcnt) {
         if (cnt > 0) atomicMax(&a.max_counts[0], cnt);
         if (gcnt > 0) atomicMax(&a.max_counts[1], gcnt);
     }
+}
+
+// First of this thread's own slots, own of them: the block takes its slots
+// with one atomic (which block gets which slots is only an address).  All 256
+// threads of the block call it.
+__device__ inline uint32_t face_slots(unsigned long long *nfaces, int own) {
+    __shared__ uint32_t wsum[4];
+    __shared__ uint32_t sbase;
+    const int lane = __lane_id(), w = threadIdx.x >> 6;
+    uint32_t incl = (uint32_t)own;
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t o = __shfl_up(incl, off, 64);
+        incl += lane >= off ? o : 0u;
+    }
+    if (lane == 63) wsum[w] = incl;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const uint32_t tot = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+        sbase = tot ? (uint32_t)atomicAdd(nfaces, (unsigned long long)tot) : 0u;
+    }
+    __syncthreads();
+    uint32_t base = sbase + incl - (uint32_t)own;
+    for (int k = 0; k < w; ++k) base += wsum[k];
+    return base;
 }
 
 // The periodic image search, on a stream of its own beside k_neighbours: a
@@ -656,12 +695,15 @@ template <int D, bool kCaller, int kDens>
 __global__ __launch_bounds__(256) void k_images_finish(NbrArgs a) {
     using TW = typename std::conditional<kDens == 4, float, double>::type;
     const int t = xcd_block() * blockDim.x + threadIdx.x;
-    int gcnt = 0;
-    if (t < a.N && a.nog[t] < 0) {
+    int gcnt = 0, own = 0;
+    const bool marked = t < a.N && a.nog[t] < 0;
+    uint16_t *rec = a.face_rec + (size_t)(marked ? t : 0) * FaceRec<D>::N;
+    if (marked) {
         const Geom &g = a.g;
         const int N = a.N, cnt = a.noi[t], src = a.img_base;
         gcnt = a.img_cnt[t];
         a.nog[t] = gcnt;
+        own = cnt + gcnt - (a.all_own ? 0 : (int)rec[2]);
         const double4 pi = a.pos_w[t];
         const double xi[3] = {pi.x, pi.y, pi.z};
         const TW wh2 = TW(g.h / 2.), wsig = TW(g.sigma);
@@ -704,6 +746,11 @@ __global__ __launch_bounds__(256) void k_images_finish(NbrArgs a) {
         }
     }
     reduce_max_counts(a, 0, gcnt);
+    if (__syncthreads_or(marked)) {
+        const uint32_t slot =
+            face_slots(a.nfaces, own) - (marked && !a.all_own ? (uint32_t)rec[2] : 0u);
+        if (marked) __builtin_memcpy(rec, &slot, 4);
+    }
 }
 
 // kDens: 0, or the bytes of the primitive records (4, 8) when the step's
@@ -711,20 +758,28 @@ __global__ __launch_bounds__(256) void k_images_finish(NbrArgs a) {
 // position, candidates from global memory: caller order and linear keys.
 template <int D, bool kCaller, int kDens>
 __global__ __launch_bounds__(256) void k_neighbours(NbrArgs a) {
+    constexpr int RN = FaceRec<D>::N;
     __shared__ __align__(16) uint32_t s_stage[256 * 16];
+    __shared__ __align__(16) uint16_t s_segs[256 * RN];
     const int t = xcd_block() * blockDim.x + threadIdx.x;
-    int cnt = 0;
+    uint16_t *segs = s_segs + RN * threadIdx.x;
+    int cnt = 0, own = 0;
     if (t < a.N) {
         const GlobalCand src{(const char *)a.pos_cell, a.cstart, a.cend};
-        search_one<D, kCaller, kDens>(a, t, src, s_stage + 16 * threadIdx.x, cnt);
+        search_one<D, kCaller, kDens>(a, t, src, s_stage + 16 * threadIdx.x, segs, cnt, own);
     }
     reduce_max_counts(a, cnt, 0);
+    const uint32_t slot = face_slots(a.nfaces, own) - (a.all_own ? 0u : (uint32_t)segs[2]);
+    __builtin_memcpy(segs, &slot, 4);
+    if (t < a.N)
+        __builtin_memcpy(__builtin_assume_aligned(a.face_rec + (size_t)t * RN, 16),
+                         __builtin_assume_aligned(segs, 16), RN * sizeof(uint16_t));
 }
 
 template __global__ void k_assign_cells<2>(Geom, const double *, const double *, const double *,
-                                           int, uint32_t *, uint32_t *);
+                                           int, uint32_t *, uint32_t *, unsigned long long *);
 template __global__ void k_assign_cells<3>(Geom, const double *, const double *, const double *,
-                                           int, uint32_t *, uint32_t *);
+                                           int, uint32_t *, uint32_t *, unsigned long long *);
 // ------------------------------------------------------------ domain limits
 // Particles::getDomainLimits (Particles.cpp:228-268) as the reference runs
 // it, sequentially per axis: min starts at DBL_MAX, max at DBL_MIN (the
@@ -881,12 +936,12 @@ __global__ void k_pack_pos(const double *__restrict__ x0, const double *__restri
 void launch_cells(const Geom &g, int D, const double *x0, const double *x1,
                   const double *x2, int N, double4 *pos, uint32_t *key, uint32_t *idx,
                   uint32_t *skey, uint32_t *scratch, int *cstart, int *cend, uint32_t *inv,
-                  hipStream_t s) {
+                  unsigned long long *nfaces, hipStream_t s) {
     int nb = (N + 255) / 256;
     if (D == 2)
-        hipLaunchKernelGGL(k_assign_cells<2>, dim3(nb), dim3(256), 0, s, g, x0, x1, x2, N, key, idx);
+        hipLaunchKernelGGL(k_assign_cells<2>, dim3(nb), dim3(256), 0, s, g, x0, x1, x2, N, key, idx, nfaces);
     else
-        hipLaunchKernelGGL(k_assign_cells<3>, dim3(nb), dim3(256), 0, s, g, x0, x1, x2, N, key, idx);
+        hipLaunchKernelGGL(k_assign_cells<3>, dim3(nb), dim3(256), 0, s, g, x0, x1, x2, N, key, idx, nfaces);
     // sort a copy: key[i] stays the cell of particle i
     hipMemcpyAsync(skey, key, sizeof(uint32_t) * N, hipMemcpyDeviceToDevice, s);
     int bits = 1;

@@ -212,6 +212,43 @@ struct FRec {
     static constexpr int N = NF * D + D * D;   // 12 (2D) / 24 (3D)
 };
 
+// Face-slot record of one work position (uint16 words, 16-byte aligned): the
+// step evaluates a real pair once, from the particle whose row lists the
+// other after its own place in the stencil order (a row is therefore [mirrored
+// entries | own entries | images]).  Words 0-1: slot of row entry 0, counted
+// back from the first own face's (modulo 2^32): row entry n >= nb has the slot
+// n after it; word 2: nb, the count of mirrored entries; word 2 + s, s =
+// 1..C: row entry where stencil cell C + s begins (C = (3^D - 1) / 2, the
+// particle's cell).  Words of cells without candidates are not set.
+template <int D>
+struct FaceRec {
+    static constexpr int C = D == 2 ? 4 : 13;
+    static constexpr int N = D == 2 ? 8 : 16;
+};
+// rows longer than this do not fit the record's words
+constexpr int kFaceRecMaxRow = 65535;
+
+// place s of cell key kt in the stencil of cell key kq, relative to the
+// middle (0: the same cell, > 0: after it); the cells are at most one apart
+template <int D>
+__device__ inline int stencil_place(const Geom &g, uint32_t kt, uint32_t kq) {
+    int d[3];
+    if (g.mbits) {
+        // masked Morton keys compare as the coordinates do
+        const uint32_t m0 = D == 2 ? 0x55555555u : 0x09249249u;
+        for (int a = 0; a < D; ++a) {
+            const uint32_t t = kt & (m0 << a), q = kq & (m0 << a);
+            d[a] = (int)(t > q) - (int)(t < q);
+        }
+    } else {
+        int ct[3], cq[3];
+        cell_coords<D>(g, kt, ct);
+        cell_coords<D>(g, kq, cq);
+        for (int a = 0; a < D; ++a) d[a] = ct[a] - cq[a];
+    }
+    return D == 2 ? 3 * d[0] + d[1] : 9 * d[0] + 3 * d[1] + d[2];
+}
+
 __device__ inline int lane_id() { return __lane_id(); }
 
 // LDS written by some lanes of a wavefront, then read by others: a
@@ -220,6 +257,21 @@ __device__ inline void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// every load to LDS of the wavefront has landed (and is seen by its reads), but
+// for its Newer latest vector memory instructions
+template <int Newer = 0>
+__device__ inline void wave_loads_done() {
+    static_assert(Newer < 16, "vmcnt's low field");
+    __builtin_amdgcn_s_waitcnt(0x0f70 | Newer);  // vmcnt(Newer)
+    wave_lds_sync();
+}
+// every LDS read of the wavefront has its data: what was read may be
+// overwritten by loads to LDS
+__device__ inline void wave_lds_reads_done() {
+    wave_lds_sync();
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
 }
 
 // XCD-aware block index.  Workgroups are dispatched round-robin over the 8

@@ -36,15 +36,12 @@ void launch_dt_finalize(const HydroArgs &a, double dt_fixed, double t_now, doubl
                        dt_fixed, t_now, t_clip, dt_in, a.dt, dt_hist, step, a.status);
 }
 void launch_faces(const HydroArgs &a, int D, int precision, hipStream_t s) {
-    dim3 grid((a.N + 255) / 256);
     if (precision != 0) {
         launch_faces_fp32(a, D, s);
-    } else if (a.learned) {
-        if (D == 2) hipLaunchKernelGGL((k_faces<2, double, true>), grid, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((k_faces<3, double, true>), grid, dim3(256), 0, s, a);
+    } else if (D == 2) {
+        launch_faces_of<2, double>(a, s);
     } else {
-        if (D == 2) hipLaunchKernelGGL((k_faces<2, double, false>), grid, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((k_faces<3, double, false>), grid, dim3(256), 0, s, a);
+        launch_faces_of<3, double>(a, s);
     }
 }
 void launch_riemann_flux(const HydroArgs &a, int D, long long n, const double *wl,

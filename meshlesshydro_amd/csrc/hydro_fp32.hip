@@ -25,16 +25,10 @@ void launch_gradients_fp32(const HydroArgs &a, int D, hipStream_t s) {
 }
 
 void launch_faces_fp32(const HydroArgs &a, int D, hipStream_t s) {
-    dim3 grid((a.N + 255) / 256);
-    if (a.learned) {
-        // faces whose standard guess was far off are solved after the row
-        // from the network's seed, inside the same kernel
-        if (D == 2) hipLaunchKernelGGL((k_faces<2, float, true>), grid, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((k_faces<3, float, true>), grid, dim3(256), 0, s, a);
-    } else {
-        if (D == 2) hipLaunchKernelGGL((k_faces<2, float, false>), grid, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((k_faces<3, float, false>), grid, dim3(256), 0, s, a);
-    }
+    // learned: faces whose standard guess was far off are solved after the
+    // row from the network's seed, inside the same kernel
+    if (D == 2) launch_faces_of<2, float>(a, s);
+    else launch_faces_of<3, float>(a, s);
 }
 
 void launch_stage_fp32(const HydroArgs &a, int D, int op, int what, const FaceArrays &fa,

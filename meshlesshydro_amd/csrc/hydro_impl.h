@@ -589,7 +589,8 @@ template <int D, typename T>
 struct View {
     static constexpr int NP = kPrimN, NFR = FRec<D>::N;
     double x[3];
-    T p[NP];
+    int i;  // original index
+    alignas(16) T p[NP];
     T f[NFR];
 };
 template <int D, typename T>
@@ -597,6 +598,7 @@ __device__ inline View<D, T> make_view(const HydroArgs &a, int j) {
     View<D, T> v;
     double4 q = a.pos[j];
     v.x[0] = q.x; v.x[1] = q.y; v.x[2] = q.z;
+    v.i = (int)q.w;
     load_vec<T, View<D, T>::NP>(v.p, (const T *)a.prim + (size_t)j * kPrimN);
     load_vec<T, View<D, T>::NFR>(v.f, (const T *)a.frec + (size_t)j * FRec<D>::N);
     return v;
@@ -1018,6 +1020,19 @@ __device__ inline void face_of_entry(const HydroArgs &a, int t, int i, int n, T 
     face_of_entry<D, T>(a, t, i, e, (int)a.pos[nb_index(e)].w, dt, fp, mp, self_lo, fs);
 }
 
+// FP64 learned: the network runs for faces with a real jump (near-uniform
+// faces keep the standard guess, which is converged to O(jump^2) there):
+// |dp| > k (pL + pR) or du^2 rhoR rhoL > 2 k^2 gamma (pR rhoL + pL rhoR)
+template <int D, typename T>
+__device__ inline bool strong_jump(const HydroArgs &a, const FacePrep<D, T> &fp) {
+    T dp = fp.WR[1] - fp.WL[1], du = fp.uj - fp.ui;
+    T psum = fp.WR[1] + fp.WL[1];
+    T rr = fp.WR[0] * fp.WL[0];
+    T c2r = T(a.gamma) * (fp.WR[1] * fp.WL[0] + fp.WL[1] * fp.WR[0]);
+    return dp * dp > T(kSeedJump * kSeedJump) * psum * psum ||
+           du * du * rr > T(2 * kSeedJump * kSeedJump) * c2r;
+}
+
 // Network seed for this lane's face when want; every lane of the wavefront
 // calls it together (BF16 MFMA over the wavefront's 64 faces).
 template <int D, typename T>
@@ -1070,22 +1085,50 @@ __device__ inline void collect_faces(const HydroArgs &a, bool want, const FacePr
     }
 }
 
-// solve the face, add its flux (with the sign of this side) to the sums;
-// face collection for the training data
+// solve the face: its flux F as the solving side sees it; face collection
+// for the training data
+template <int D, typename T>
+__device__ inline void face_flux(const HydroArgs &a, const FacePrep<D, T> &fp,
+                                 const MixedProbe &mp, float seed, int it0, bool collect, T *F,
+                                 FaceStats &fs) {
+    face_finish<D, T>(a, fp, seed, F, fs, sizeof(T) == 4 ? &mp : nullptr);
+    if (a.collect) collect_faces<D, T>(a, collect && fs.st.iters - it0 >= 2, fp);
+}
+
+// ... added to the sums with the sign of this side
 template <int D, typename T>
 __device__ inline void face_accumulate(const HydroArgs &a, const FacePrep<D, T> &fp,
                                        const MixedProbe &mp, float seed, bool self_lo, int it0,
                                        bool collect, FluxSums &acc, FaceStats &fs) {
     T F[D + 2];
-    face_finish<D, T>(a, fp, seed, F, fs, sizeof(T) == 4 ? &mp : nullptr);
-    if (a.collect) collect_faces<D, T>(a, collect && self_lo && fs.st.iters - it0 >= 2, fp);
+    face_flux<D, T>(a, fp, mp, seed, it0, collect && self_lo, F, fs);
     double sgn = self_lo ? 1. : -1.;
     acc.m += sgn * (double)F[0];
     for (int ax = 0; ax < D; ++ax) acc.v[ax] += sgn * (double)F[2 + ax];
     acc.e += sgn * (double)F[1];
 }
 
-
+__device__ inline void add_stats(FaceStats &fs, const FaceStats &o) {
+    fs.neg_real += o.neg_real;
+    fs.neg_ghost += o.neg_ghost;
+    fs.vacuum += o.vacuum;
+    fs.seeded += o.seeded;
+    fs.st.iters += o.st.iters;
+    fs.st.fallback += o.st.fallback;
+    fs.st.nonconv += o.st.nonconv;
+    fs.st.acoustic += o.st.acoustic;
+}
+// counters of faces that stand for both of their directed entries
+__device__ inline void double_stats(FaceStats &fs) {
+    fs.neg_real *= 2;
+    fs.neg_ghost *= 2;
+    fs.vacuum *= 2;
+    fs.seeded *= 2;
+    fs.st.iters *= 2;
+    fs.st.fallback *= 2;
+    fs.st.nonconv *= 2;
+    fs.st.acoustic *= 2;
+}
 
 // the state of particle i carried over unchanged (a step whose neighbour
 // search overflowed)
@@ -1171,7 +1214,8 @@ __device__ inline void add_counters(const HydroArgs &a, const FaceStats fs, int 
 #define MLH_FACES_WAVES(D, T, LEARNED) ((LEARNED && sizeof(T) == 4) ? 2 : 1)
 #endif
 
-// Faces of particle i.  LEARNED: the loop runs to the wavefront's largest
+// Faces of particle i, every one of its row evaluated here, where the fluxes
+// of k_face_pairs have no room.  LEARNED: the loop runs to the wavefront's largest
 // neighbour count so that every lane takes part in the BF16 MFMA inference
 // of the p* seed for the wavefront's 64 faces of that iteration.
 template <int D, typename T, bool LEARNED>
@@ -1189,6 +1233,7 @@ __attribute__((amdgpu_waves_per_eu(MLH_FACES_WAVES(D, T, LEARNED)))) void k_face
     const bool live = t < a.N;
     FaceStats fs{};
     const int N = a.N;
+    if (a.flux && *a.nfaces <= a.fcap) return;  // k_face_pairs and k_face_sum did it all
     const int i = live ? (a.sidx ? (int)a.sidx[t] : t) : 0;
     if (a.status[0] & kStatusErrMask) {
         // this step's neighbour search overflowed (the reference exits in
@@ -1237,19 +1282,7 @@ __attribute__((amdgpu_waves_per_eu(MLH_FACES_WAVES(D, T, LEARNED)))) void k_face
         if (act) face_of_entry<D, T>(a, t, i, e, jo, dt, fp, mp, self_lo, fs, kOwnView ? &own : nullptr);
         float seed = -1.f;
         if constexpr (kInLoopNet) {
-            // FP64: the network runs for faces with a real jump
-            // (near-uniform faces keep the standard guess, which is converged
-            // to O(jump^2) there): |dp| > k (pL + pR) or
-            // du^2 rhoR rhoL > 2 k^2 gamma (pR rhoL + pL rhoR)
-            bool strong = false;
-            if (act) {
-                T dp = fp.WR[1] - fp.WL[1], du = fp.uj - fp.ui;
-                T psum = fp.WR[1] + fp.WL[1];
-                T rr = fp.WR[0] * fp.WL[0];
-                T c2r = T(a.gamma) * (fp.WR[1] * fp.WL[0] + fp.WL[1] * fp.WR[0]);
-                strong = dp * dp > T(kSeedJump * kSeedJump) * psum * psum ||
-                         du * du * rr > T(2 * kSeedJump * kSeedJump) * c2r;
-            }
+            const bool strong = act && strong_jump<D, T>(a, fp);
             if (__ballot(strong)) seed = face_net_seed<D, T>(a, strong, fp, lds[threadIdx.x >> 6], fs);
         }
         if (act) {
@@ -1325,6 +1358,448 @@ __attribute__((amdgpu_waves_per_eu(MLH_FACES_WAVES(D, T, LEARNED)))) void k_face
     add_counters(a, fs, cnt);
 }
 
+// Views in LDS, 16-byte chunk by chunk: chunk c of the neighbour of lane l and
+// of particle p of the wavefront's group lie at (64 + G) c + l and (64 + G) c +
+// 64 + p, so that one per-lane place serves all chunks of either, and a chunk
+// of the 64 neighbours is what one direct load to LDS fills.  Chunks: position
+// and original index (double4), primitive record, face record.
+template <int D, typename T, int G>
+struct FaceLds {
+    static constexpr int kPos = 2, kPrim = kPrimN * (int)sizeof(T) / 16;
+    static constexpr int kFrec = FRec<D>::N * (int)sizeof(T) / 16;
+    static constexpr int kChunks = kPos + kPrim + kFrec, kRow = 64 + G;
+    float4 v[kChunks * kRow];
+    // The real (phase 0) or image (phase 1) faces of the group as one list:
+    // particle by particle, each in row order, so that every lane has a face
+    // until the list ends, however the particles' counts differ.
+    int pre[G + 1];     // list place of each particle's first face, the end
+    int row0[G];        // row entry of that face
+    uint32_t slot0[G];  // slot of row entry 0 (modulo 2^32)
+};
+struct FaceCursor {
+    int p, g;  // particle in the group, list place
+};
+struct FaceCounts {
+    int nr, ng, nb;     // this lane's particle: real, image, mirrored entries
+};
+
+typedef __attribute__((address_space(3))) float4 lds_float4;
+typedef __attribute__((address_space(1))) const float4 global_float4;
+
+// the chunks of the records of position q to the places of lane l (off = 0) or
+// of particle l (off = 64), for the active lanes; complete when the wavefront's
+// loads are (face_view's reads wait for them)
+template <int D, typename T, int G>
+__device__ inline void face_fetch(const HydroArgs &a, int q, int off, FaceLds<D, T, G> &g) {
+    using L = FaceLds<D, T, G>;
+    const float4 *src[3] = {(const float4 *)(a.pos + q),
+                            (const float4 *)((const T *)a.prim + (size_t)q * kPrimN),
+                            (const float4 *)((const T *)a.frec + (size_t)q * FRec<D>::N)};
+    constexpr int len[3] = {L::kPos, L::kPrim, L::kFrec};
+    int c = 0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+        for (int u = 0; u < len[k]; ++u, ++c)
+            __builtin_amdgcn_global_load_lds((global_float4 *)(src[k] + u),
+                                             (lds_float4 *)&g.v[c * L::kRow + off], 16, 0, 0);
+}
+// the view at place l
+template <int D, typename T, int G>
+__device__ inline void face_view(const FaceLds<D, T, G> &g, int place, View<D, T> &v) {
+    using L = FaceLds<D, T, G>;
+    float4 r[L::kChunks];
+#pragma unroll
+    for (int c = 0; c < L::kChunks; ++c) r[c] = g.v[c * L::kRow + place];
+    double x[4];
+    __builtin_memcpy(x, r, 32);
+    v.x[0] = x[0]; v.x[1] = x[1]; v.x[2] = x[2];
+    v.i = (int)x[3];
+    __builtin_memcpy(v.p, r + L::kPos, sizeof(v.p));
+    __builtin_memcpy(v.f, r + L::kPos + L::kPrim, sizeof(v.f));
+}
+
+// every lane of the wavefront calls these
+template <int D, typename T, int G>
+__device__ inline FaceCounts group_load(const HydroArgs &a, int t0, FaceLds<D, T, G> &g) {
+    FaceCounts c{0, 0, 0};
+    const int lane = lane_id(), t = t0 + lane;
+    if (lane < a.face_group && t < a.N) {
+        c.nr = a.noi[t];
+        c.ng = a.nog[t];
+        const uint16_t *rec = a.face_rec + (size_t)t * FaceRec<D>::N;
+        __builtin_memcpy(&g.slot0[lane], rec, 4);
+        c.nb = a.enforce_flux_sym ? (int)rec[2] : 0;
+        face_fetch<D, T, G>(a, t, 64, g);
+    }
+    return c;
+}
+// the list of a phase; returns its length
+template <int D, typename T, int G>
+__device__ inline int group_list(const FaceCounts &c, int phase, FaceLds<D, T, G> &g) {
+    const int lane = lane_id();
+    int incl = phase == 0 ? c.nr - c.nb : c.ng;
+    for (int off = 1; off < G; off <<= 1) {
+        const int o = __shfl_up(incl, off, 64);
+        incl += lane >= off ? o : 0;
+    }
+    wave_lds_sync();
+    if (lane < G) {
+        g.pre[lane + 1] = incl;
+        g.row0[lane] = phase == 0 ? c.nb : c.nr;
+    }
+    if (lane == 0) g.pre[0] = 0;
+    wave_lds_sync();
+    return g.pre[G];
+}
+// moves the cursor on by step places, at most to the end; false there
+template <int D, typename T, int G>
+__device__ inline bool cursor_next(const FaceLds<D, T, G> &g, FaceCursor &c, int step, int total) {
+    c.g += step;
+    if (c.g >= total) {
+        c.g = total;
+        return false;
+    }
+    while (c.g >= g.pre[c.p + 1]) ++c.p;
+    return true;
+}
+template <int D, typename T, int G>
+__device__ inline int cursor_entry(const FaceLds<D, T, G> &g, const FaceCursor &c) {
+    return g.row0[c.p] + (c.g - g.pre[c.p]);
+}
+template <int D, typename T, int G>
+__device__ inline T *cursor_slot(const HydroArgs &a, const FaceLds<D, T, G> &g, const FaceCursor &c) {
+    return (T *)a.flux + (size_t)(g.slot0[c.p] + (uint32_t)cursor_entry(g, c)) * (D + 2);
+}
+// the face of row entry e of the group's particle p, whose neighbour's records
+// are at this lane's place, solved from the lower original index (images:
+// parent >= i); recorded: a training face of its solving particle.  FP32: also
+// the first step of the mixed solver.  read: called once the two views are in
+// registers.  Every lane of the wavefront calls this, act for those with a face.
+template <int D, typename T, int G, typename Read>
+__device__ inline void group_face(const HydroArgs &a, const FaceLds<D, T, G> &g, bool act, int p,
+                                  uint32_t e, bool image, T dt, FacePrep<D, T> &fp, MixedProbe &mp,
+                                  bool &self_lo, bool &recorded, FaceStats &fs, Read &&read) {
+    using LS = FaceLds<D, T, G>;
+    int s[3] = {0, 0, 0};
+    if (image)
+        for (int ax = 0; ax < D; ++ax) s[ax] = code_shift(nb_code(e), ax);
+    const int po = 64 + p, pn = lane_id();
+    const int i = (int)((const double *)&g.v[LS::kRow + po])[1];
+    const int jo = (int)((const double *)&g.v[LS::kRow + pn])[1];
+    const bool sym = a.enforce_flux_sym;
+    self_lo = !sym || (image ? jo >= i : jo > i);
+    recorded = a.collect && (image || !sym ? self_lo && i % a.collect_stride == 0
+                                           : (self_lo ? i : jo) % a.collect_stride == 0);
+    View<D, T> L, H;
+    face_view<D, T, G>(g, self_lo ? po : pn, L);
+    face_view<D, T, G>(g, self_lo ? pn : po, H);
+    read();
+    if (!act) return;
+    int sl[3];
+    for (int ax = 0; ax < 3; ++ax) sl[ax] = self_lo ? s[ax] : -s[ax];
+    face_prepare<D, T>(a, L, H, sl, image, dt, fp, fs);
+    if constexpr (sizeof(T) == 4) mp = face_probe<D>(a, fp, fs.st);
+}
+
+// FP32 learned: the mass flux of a face left to k_face_deferred (a NaN that
+// no arithmetic makes), in its slot until then
+constexpr uint32_t kDeferredTag = 0x7fc5eed1u;
+
+// Each real face once, from the particle that lists the other after its own
+// place in the stencil order (FaceRec), and the images: the flux as that
+// particle sees it goes to the face's slot (k_face_sum adds it to both).
+// One wavefront per block, face_group particles each: their views are held in
+// LDS, their faces dealt to the lanes as one list.  The records of a round's 64
+// neighbours go straight to LDS while the round before is being solved.
+// Bound by VALU issue (FP32) and by the latency of dependent FP64 operations at
+// one wavefront per SIMD (FP64, 304 registers; held to 256 it spills and takes
+// 8.4 ms instead of 7.3 at 128^3).  The list, not a row per lane, because own
+// faces per particle differ (11 to 45 on a lattice with 28 on average: a row
+// per lane took 2.20 ms in FP32, the list 1.74, with direct loads to LDS 1.45);
+// the rows are shared out by one wavefront so that the stores of a round are
+// side by side (scattered by row they took the kernel to 3.17 ms).
+// With k_face_sum, 128^3 blast: 2.77 -> 1.45 + 1.27 ms FP32, 12.24 -> 7.29 +
+// 1.58 ms FP64; turbulent box 160^3 FP32 12.9 -> 6.5 + 3.0 ms; 100^2 shear FP64
+// 296 -> 63 + 14 us (k_faces evaluates each face from both sides).
+// LEARNED: in FP64 the network runs in the loop; in FP32 a face whose standard
+// guess was far off is left to k_face_deferred, its round listed in a.deferred
+// ([0].x the length, then {group, phase << 31 | round}).
+template <int D, typename T, bool LEARNED, int G>
+__global__ __launch_bounds__(64)
+__attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 2 : 1))) void k_face_pairs(HydroArgs a) {
+    constexpr int NF = D + 2;
+    constexpr bool kInLoopNet = LEARNED && sizeof(T) == 8;
+    constexpr bool kDefer = LEARNED && sizeof(T) == 4;
+    __shared__ FaceLds<D, T, G> g;
+    __shared__ uint16_t s_net[kInLoopNet ? 64 * 16 : 1];
+    if (*a.nfaces > a.fcap || (a.status[0] & kStatusErrMask)) return;
+    const int lane = lane_id();
+    const int group = xcd_block(), t0 = group * a.face_group;
+    const T dt = T(a.dt[0]);
+    const FaceCounts cn = group_load<D, T, G>(a, t0, g);
+    FaceStats fs{};
+    for (int phase = 0; phase < 2; ++phase) {
+        if (phase == 1 && !__ballot(cn.ng > 0)) break;
+        const int total = group_list<D, T, G>(cn, phase, g);
+        // row entries two rounds ahead, the neighbours' records one
+        FaceCursor c0{0, lane}, c1, c2;
+        uint32_t e0 = 0, e1 = 0;
+        auto load = [&](const FaceCursor &c) { return nb_get(a.nbr, a.N, t0 + c.p, cursor_entry(g, c)); };
+        if (cursor_next(g, c0, 0, total)) {
+            e0 = load(c0);
+            face_fetch<D, T, G>(a, (int)nb_index(e0), 0, g);
+        }
+        c1 = c0;
+        if (cursor_next(g, c1, 64, total)) e1 = load(c1);
+        c2 = c1;
+        wave_loads_done();  // the first round's records
+        for (int left = total; left > 0; left -= 64) {
+            const bool act = c0.g < total;
+            // this round's records; the flux stores behind them (16 bytes at
+            // most per instruction) may be under way
+            if (left < total) wave_loads_done<(NF * (int)sizeof(T) + 15) / 16>();
+            uint32_t e2 = 0;
+            if (cursor_next(g, c2, 64, total)) e2 = load(c2);
+            FacePrep<D, T> fp;
+            MixedProbe mp{};
+            bool self_lo = true, recorded = false;
+            const int it0 = fs.st.iters;
+            group_face<D, T, G>(a, g, act, c0.p, e0, phase == 1, dt, fp, mp, self_lo, recorded, fs, [&] {
+                // the views have been read: the next round's records
+                wave_lds_reads_done();
+                if (c1.g < total) face_fetch<D, T, G>(a, (int)nb_index(e1), 0, g);
+            });
+            float seed = -1.f;
+            if constexpr (kInLoopNet) {
+                const bool strong = act && strong_jump<D, T>(a, fp);
+                if (__ballot(strong)) seed = face_net_seed<D, T>(a, strong, fp, s_net, fs);
+            }
+            bool far = false;
+            if (act) {
+                // a deferred face goes on with A = 0, for which face_finish
+                // returns zero flux at once: one path for every face
+                far = kDefer && mp.valid && !mp.accepted && mp.chg > kSeedGate;
+                if (far)
+                    for (int ax = 0; ax < D; ++ax) fp.A[ax] = T(0);
+                T F[NF];
+                face_flux<D, T>(a, fp, mp, seed, it0, recorded, F, fs);
+                if constexpr (kDefer)
+                    if (far) {
+                        F[0] = __uint_as_float(kDeferredTag);
+                        self_lo = true;
+                    }
+                T *dst = cursor_slot(a, g, c0);
+                for (int k = 0; k < NF; ++k) dst[k] = self_lo ? F[k] : -F[k];
+            }
+            if constexpr (kDefer)
+                if (__ballot(far) && lane == 0)
+                    a.deferred[1 + atomicAdd(&a.deferred[0].x, 1u)] =
+                        make_uint2((uint32_t)group, (uint32_t)phase << 31 | (uint32_t)(total - left) / 64);
+            c0 = c1;
+            e0 = e1;
+            c1 = c2;
+            e1 = e2;
+        }
+        if (phase == 0 && a.enforce_flux_sym) double_stats(fs);
+    }
+    add_counters(a, fs, cn.nr + cn.ng);
+}
+
+// FP32 learned: the tagged faces of the listed rounds, Newton from the
+// network's seed, one round per block at a time.  Whether a face is deferred
+// depends on the face alone (the probe runs on the solving side's operands).
+// Every lane takes part in the round's BF16 MFMA inference.
+template <int D, int G>
+__global__ __launch_bounds__(64) void k_face_deferred(HydroArgs a) {
+    constexpr int NF = D + 2;
+    __shared__ FaceLds<D, float, G> g;
+    __shared__ uint16_t s_net[64 * 16];
+    if (*a.nfaces > a.fcap || (a.status[0] & kStatusErrMask)) return;
+    const float dt = (float)a.dt[0];
+    const uint32_t rounds = a.deferred[0].x;
+    FaceStats fs{};
+    for (uint32_t k = blockIdx.x; k < rounds; k += gridDim.x) {
+        const uint2 at = a.deferred[1 + k];
+        const int t0 = (int)at.x * a.face_group, phase = (int)(at.y >> 31);
+        const FaceCounts cn = group_load<D, float, G>(a, t0, g);
+        const int total = group_list<D, float, G>(cn, phase, g);
+        FaceCursor c{0, 0};
+        bool far = cursor_next(g, c, (int)(at.y & 0x7fffffffu) * 64 + lane_id(), total);
+        float *dst = nullptr;
+        if (far) {
+            dst = cursor_slot(a, g, c);
+            far = __float_as_uint(dst[0]) == kDeferredTag;
+        }
+        FacePrep<D, float> fp;
+        MixedProbe mp{};
+        bool self_lo = true, recorded = false;
+        FaceStats seen{}, fd{};  // the probe was counted in k_face_pairs
+        uint32_t e = 0;
+        if (far) {
+            e = nb_get(a.nbr, a.N, t0 + c.p, cursor_entry(g, c));
+            face_fetch<D, float, G>(a, (int)nb_index(e), 0, g);
+        }
+        wave_loads_done();
+        group_face<D, float, G>(a, g, far, c.p, e, phase == 1, dt, fp, mp, self_lo, recorded, seen, [] {});
+        const float seed = face_net_seed<D, float>(a, far, fp, s_net, fd);
+        if (far) {
+            float F[NF];
+            face_flux<D, float>(a, fp, mp, seed, fd.st.iters, recorded, F, fd);
+            for (int q = 0; q < NF; ++q) dst[q] = self_lo ? F[q] : -F[q];
+        }
+        if (phase == 0 && a.enforce_flux_sym) double_stats(fd);
+        add_stats(fs, fd);
+        wave_lds_reads_done();  // the next group's records go to the same places
+    }
+    add_counters(a, fs, 0);
+}
+
+// Slot of the face between work position t (cell key kt) and q, which q
+// evaluates (t lies after q in q's stencil order): the row entry of q that
+// holds t is looked for in the segment of q's row for t's cell.
+struct MirrorPlace {
+    uint32_t slot0;  // slot of q's row entry 0
+    int m;           // the row entry the segment starts at
+};
+template <int D>
+__device__ inline MirrorPlace mirror_place(const HydroArgs &a, uint32_t kt, int q) {
+    const int s = stencil_place<D>(a.g, kt, a.ck[q]);
+    const uint16_t *rec = a.face_rec + (size_t)q * FaceRec<D>::N;
+    MirrorPlace p;
+    __builtin_memcpy(&p.slot0, rec, 4);
+    p.m = s < 0 || s > FaceRec<D>::C ? kFaceRecMaxRow : (int)rec[2 + s];
+    return p;
+}
+// e: row entries m & ~3 .. + 3 of q.  ~0u when q does not list t (an
+// overflowed row, whose step is not used).
+__device__ inline uint32_t mirror_slot(const HydroArgs &a, int t, int q, const MirrorPlace &p,
+                                       uint32_t *e) {
+    const uint32_t want = (uint32_t)t | (kCodeReal << kIdxBits);
+    int m = p.m & ~3;
+    for (;;) {
+        const int u = e[0] == want ? 0 : e[1] == want ? 1 : e[2] == want ? 2 : e[3] == want ? 3 : 4;
+        if (u < 4) {
+            const uint32_t slot = p.slot0 + (uint32_t)(m + u);
+            return slot < a.fcap ? slot : ~0u;
+        }
+        m += 4;
+        if (m >= a.maxr) return ~0u;
+        nb_get4(a.nbr, a.N, q, m, e);
+    }
+}
+// the entries of q's row the search starts with (entry 0 for a place past it)
+__device__ inline void mirror_row(const HydroArgs &a, int q, const MirrorPlace &p, uint32_t *e) {
+    nb_get4(a.nbr, a.N, q, p.m < a.maxr ? p.m & ~3 : 0, e);
+}
+
+// The flux sums of the particles from the stored faces, in row order (the
+// reference's collectFluxes order), and the update.  A mirrored entry takes
+// the partner's flux with the opposite sign, so F_ji = -F_ij bitwise.
+// Bound by the L1's cache accesses: the lookups take about 0.6 of its 1.27 ms
+// at 128^3 FP32, the fluxes 0.4, the state 0.25.  One thread per particle took
+// 2.4 ms: 64 rows of slots in flight per wavefront push each other out of L2.
+// Eight lanes per particle and sixteen entries at a time: each lane looks up
+// and loads the fluxes of two entries, then (through LDS) lane c sums
+// component c of the sixteen in entry order.
+constexpr int kSumLanes = 8;
+template <int D, typename T>
+__global__ __launch_bounds__(256) void k_face_sum(HydroArgs a) {
+    constexpr int NF = D + 2, P = 256 / kSumLanes, U = 2, B = U * kSumLanes;
+    __shared__ T s_flux[P][B][NF];
+    __shared__ double s_sum[P][NF];
+    if (*a.nfaces > a.fcap) return;
+    const int b0 = xcd_block() * P, N = a.N;
+    const int p = (int)(threadIdx.x / kSumLanes), l = (int)(threadIdx.x & (kSumLanes - 1));
+    const int t = b0 + p;
+    if (a.deferred && b0 == 0 && threadIdx.x == 0) a.deferred[0].x = 0;  // for the next step
+    if (!(a.status[0] & kStatusErrMask)) {
+        const bool live = t < N;
+        const int cnt = live ? a.noi[t] + a.nog[t] : 0;
+        const uint32_t kt = live ? a.ck[t] : 0u;
+        const uint16_t *rec = a.face_rec + (size_t)(live ? t : 0) * FaceRec<D>::N;
+        uint32_t slot0;
+        __builtin_memcpy(&slot0, rec, 4);
+        const int nb = a.enforce_flux_sym ? (int)rec[2] : 0;
+        const T *flux = (const T *)a.flux;
+        T(*fx)[NF] = s_flux[p];
+        double acc = 0.;
+        for (int n = 0; n < cnt; n += B) {
+            const int m0 = n + l;
+            uint32_t slot[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int m = m0 + u * kSumLanes;
+                slot[u] = m >= nb && m < cnt ? slot0 + (uint32_t)m : ~0u;
+            }
+            if (m0 < nb) {
+                // the lane's mirrored entries, each of the lookup's loads in
+                // flight for all of them
+                int q[U];
+                MirrorPlace mp[U];
+                uint32_t er[U][4];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int m = m0 + u * kSumLanes;
+                    q[u] = (int)nb_index(nb_get(a.nbr, N, t, m < nb ? m : m0));
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) mp[u] = mirror_place<D>(a, kt, q[u]);
+#pragma unroll
+                for (int u = 0; u < U; ++u) mirror_row(a, q[u], mp[u], er[u]);
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (m0 + u * kSumLanes < nb) slot[u] = mirror_slot(a, t, q[u], mp[u], er[u]);
+            }
+            T f[U][NF];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                __builtin_memcpy(f[u], flux + (size_t)(slot[u] != ~0u ? slot[u] : 0u) * NF, sizeof(f[u]));
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                for (int c = 0; c < NF; ++c)
+                    fx[u * kSumLanes + l][c] =
+                        slot[u] == ~0u ? T(0) : m0 + u * kSumLanes < nb ? -f[u][c] : f[u][c];
+            wave_lds_sync();
+            if (l < NF) {
+#pragma unroll
+                for (int k = 0; k < B; ++k) acc += (double)fx[k][l];
+            }
+            wave_lds_sync();
+        }
+        if (l < NF) s_sum[p][l] = acc;
+    }
+    __syncthreads();
+    if (threadIdx.x >= P) return;
+    const int u = b0 + (int)threadIdx.x;
+    const bool live = u < N;
+    const int i = live ? (a.sidx ? (int)a.sidx[u] : u) : 0;
+    if (a.status[0] & kStatusErrMask) {
+        if (live) particle_keep<D>(a, i);
+        return;
+    }
+    int bad = 0;
+    if (live) {
+        const double *s = s_sum[threadIdx.x];
+        bad = particle_finish<D>(a, i, FluxSums{s[0], s[1], {s[2], s[3], D == 3 ? s[D + 1] : 0.}});
+    }
+    if (a.debug) {
+        const unsigned long long nf = wave_sum((unsigned long long)bad);
+        if (lane_id() == 0 && nf) atomicAdd(&a.counters[kCntNonfinite], nf);
+    }
+}
+// most particles per wavefront of k_face_pairs: as many as leave the LDS room for
+// the wavefronts the registers allow (FP32 18.5 KB: 1.50 ms at 128^3 against
+// 1.54 with 32, 1.64 with 64; FP64 28 KB: 32 and 64 alike)
+template <int D, typename T>
+constexpr int kPairGroup = sizeof(T) == 4 ? 48 : 32;
+// wavefronts k_face_pairs is given at least (down to 4 particles each): one per
+// SIMD.  100^2 shear FP64 64 us; 71 with 1536, 96 with 2048 (their lists end in
+// a third round for a few faces); 40^3 turbulence FP64 400 us, 503 with 2048
+constexpr int kPairWaves = 1024;
+// wavefronts of k_face_deferred
+constexpr int kDeferredBlocks = 2048;
+
 
 // conserved sums (Particles.cpp:2830-2886): V, M, E, px, py, pz per block
 template <int D, typename T>
@@ -1356,6 +1831,30 @@ __global__ __launch_bounds__(256) void k_sums(HydroArgs a, double *out) {
     }
     if (threadIdx.x == 0)
         for (int k = 0; k < 6; ++k) out[(size_t)blockIdx.x * 6 + k] = sh[k][0];
+}
+
+template <int D, typename T, bool LEARNED>
+static void launch_faces_as(const HydroArgs &a, hipStream_t s) {
+    const dim3 blk(256), rows((a.N + 255) / 256);
+    if (a.flux) {
+        constexpr int G = kPairGroup<D, T>;
+        HydroArgs p = a;
+        p.face_group = G;
+        if (a.N < kPairWaves * G) p.face_group = a.N / kPairWaves > 4 ? a.N / kPairWaves : 4;
+        hipLaunchKernelGGL((k_face_pairs<D, T, LEARNED, G>), dim3((a.N + p.face_group - 1) / p.face_group),
+                           dim3(64), 0, s, p);
+        if constexpr (LEARNED && sizeof(T) == 4)
+            hipLaunchKernelGGL((k_face_deferred<D, G>), dim3(kDeferredBlocks), dim3(64), 0, s, p);
+        hipLaunchKernelGGL((k_face_sum<D, T>), dim3((a.N + 256 / kSumLanes - 1) / (256 / kSumLanes)),
+                           blk, 0, s, a);
+        if (a.flux_fits) return;
+    }
+    hipLaunchKernelGGL((k_faces<D, T, LEARNED>), rows, blk, 0, s, a);
+}
+template <int D, typename T>
+static void launch_faces_of(const HydroArgs &a, hipStream_t s) {
+    if (a.learned) launch_faces_as<D, T, true>(a, s);
+    else launch_faces_as<D, T, false>(a, s);
 }
 
 }  // namespace mlh

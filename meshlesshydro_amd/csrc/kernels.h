@@ -27,6 +27,12 @@ struct NbrArgs {
     // moves them behind the real entries.
     int *img_cnt;
     int img_base;
+    // slots of the faces each particle evaluates (FaceRec), handed out block
+    // by block from the counter nfaces; all_own: every entry is evaluated
+    // from its own side (no flux symmetry enforced)
+    uint16_t *face_rec;
+    unsigned long long *nfaces;
+    int all_own;
     // The step's compDensity + compPressure fused into the search (dens =
     // 4: FP32 records, 8: FP64 records, 0: off): omega summed over the hits
     // in row order, the self term, the images in row order, then the
@@ -54,6 +60,19 @@ struct HydroArgs {
     const double4 *pos;
     const uint32_t *nbr;
     const int *noi, *nog;
+    // fluxes of the step's faces, each evaluated once (k_face_sum): slots
+    // [fcap][D+2] of T, null when every face is evaluated from both sides;
+    // *nfaces > fcap: they do not fit, and the step evaluates both sides;
+    // flux_fits: they fit whatever the neighbour lists are
+    void *flux;
+    const uint16_t *face_rec;
+    const unsigned long long *nfaces;
+    unsigned long long fcap;
+    int flux_fits;
+    int face_group;              // particles per wavefront of k_face_pairs
+    uint2 *deferred;             // FP32 learned: rounds with deferred faces
+    int maxr;
+    const uint32_t *ck;          // cell key at each work position
     // state (current) and next state
     const double *x[3], *v[3], *m, *u;
     double *xn[3], *vn[3], *mn, *un;
@@ -109,7 +128,7 @@ enum CounterIdx {
 void launch_cells(const Geom &g, int D, const double *x0, const double *x1,
                   const double *x2, int N, double4 *pos, uint32_t *key, uint32_t *idx,
                   uint32_t *skey, uint32_t *scratch, int *cstart, int *cend, uint32_t *inv,
-                  hipStream_t s);
+                  unsigned long long *nfaces, hipStream_t s);
 // returns whether the search computed the density (NbrArgs::dens): the
 // cell-order search does not, and the caller then runs the density stage
 // Row entry where the image search stores: past the sector holding the real
