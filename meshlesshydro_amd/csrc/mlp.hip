@@ -321,75 +321,257 @@ __global__ __launch_bounds__(256) void k_mlp_infer_bf16(const MlpFrags *__restri
 }
 
 // ---- batched exact Riemann solver -------------------------------------------
+// Each wavefront works through its own run of faces, 64 at a time, one per
+// lane.  A face's cost varies from none (vacuum) over 1 to 11 Newton iterations
+// to 80 (2% of random states: Newton jumps about until max_iter and is bisected),
+// and a wavefront of 64 mixed faces takes as long as its longest: 73 iterations
+// for a mean of 5.5.  So a solve stops after kCapFirst iterations (78% of
+// random states are done; FP32 mode: before any FP64 iteration) and what is
+// left waits on the wavefront's lists in LDS until 64 such faces can go on
+// together: list 0 up to kCapSecond, list 1 to the end.  FP64 issue bounds
+// it (80% of the time at three wavefronts per SIMD).
+// 2^24 random states FP64: 9.9 ms in one go, 2.2 ms; 2^26 FP32: standard seed
+// 41 -> 8.4 ms, learned seed 13.4 -> 7.5 ms.  Caps 4/11 to 6/12: 2.2 to 2.4 ms.
+// A list per block in place of one per wavefront: 2.2 ms FP64, 1.1 ms more
+// learned; the next states loaded ahead: 45 registers more, spilled.  Learned
+// seed: weights kept in registers 1 wavefront per SIMD, 14 ms; read for one
+// tile of 16 faces at a time 8.8, for two 7.9, for all four 7.5.
 // Faces the FP64 solver finished: added to fallbacks[0] (atomics), or, with
 // block_counts, block b's count stored in block_counts[b] (every block
 // stores its slot, zero included, so the slots need no clearing).
-__global__ __launch_bounds__(256) void k_riemann_batch(
-    int64_t n, double gamma, const double *__restrict__ dl, const double *__restrict__ ul,
-    const double *__restrict__ pl, const double *__restrict__ dr, const double *__restrict__ ur,
-    const double *__restrict__ pr, double *__restrict__ ds, double *__restrict__ us,
-    double *__restrict__ ps, int *__restrict__ flag, int *__restrict__ iters, int precision,
-    const MlpFrags *__restrict__ F, double tol, int max_iter, int iters32,
-    unsigned long long *__restrict__ fallbacks, double *__restrict__ pstar,
-    unsigned long long *__restrict__ block_counts) {
-    __shared__ unsigned long long wcount[4];
-    __shared__ uint16_t lds[4][64 * 16];
-    int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    bool active = k < n;
-    double a0 = active ? dl[k] : 1., a1 = active ? ul[k] : 0., a2 = active ? pl[k] : 1.;
-    double b0 = active ? dr[k] : 1., b1 = active ? ur[k] : 0., b2 = active ? pr[k] : 1.;
-    float seed = -1.f;
-    if (F) {
-        // every lane of the wavefront takes part in the MFMA inference
-        float f[kMlpIn];
-        bool ok = a0 > 0. && b0 > 0. && a2 > 0. && b2 > 0.;
-        float pref = ok ? mlp_features_fast((float)gamma, (float)a0, (float)a1, (float)a2,
-                                            (float)b0, (float)b1, (float)b2, f)
-                        : 1.f;
-        if (!ok)
-            for (int q = 0; q < kMlpIn; ++q) f[q] = 0.f;
-        MlpRegs R;
-        mlp_load_regs(F, R);
-        float y = mlp_infer_wave_bf16(R, f, lds[threadIdx.x >> 6]);
-        seed = ok ? mlp_seed_from_output(y, f, pref) : -1.f;
-    }
-    SolveStats st{};
-    if (pstar) {
-        if (!active) return;
-        GasConst<double> gc(gamma);
-        pstar[k] = star_pressure_fp64(gc, a0, a1, a2, b0, b1, b2, tol, max_iter, st);
-        if (iters) iters[k] = st.iters;
+enum { kSolveMixed = 0, kSolveFp64 = 1, kSolvePstar = 2 };
+constexpr int kCapFirst = 5, kCapSecond = 11;
+
+struct BatchArgs {
+    int64_t n;
+    int tiles;  // rounds of new faces per wavefront
+    double gamma;
+    const double *in[6];          // rhoL, uL, PL, rhoR, uR, PR
+    double *ds, *us, *ps, *pstar;
+    int *flag, *iters;
+    const MlpFrags *F;
+    double tol;
+    int max_iter, iters32;
+    unsigned long long *fallbacks, *block_counts;
+};
+
+// The network's seed of the calling lane's face (-1: none); all 64 lanes
+// together, lds: 64 * 16 of the wavefront's LDS.
+template <int U>
+__device__ inline float batch_seed(const BatchArgs &a, double dl, double ul, double pl, double dr,
+                                   double ur, double pr, uint16_t *lds) {
+    float f[kMlpIn];
+    // gamma's quotients stay where they are: hoisted out of a loop, the
+    // compiler divides with other roundings
+    float gamma = (float)a.gamma;
+    asm volatile("" : "+v"(gamma));
+    const bool ok = dl > 0. && dr > 0. && pl > 0. && pr > 0.;
+    const float pref = ok ? mlp_features_fast(gamma, (float)dl, (float)ul, (float)pl, (float)dr,
+                                              (float)ur, (float)pr, f)
+                          : 1.f;
+    if (!ok)
+        for (int q = 0; q < kMlpIn; ++q) f[q] = 0.f;
+    const float y = mlp_infer_wave_bf16_lean<U>(a.F, f, lds);
+    return ok ? mlp_seed_from_output(y, f, pref) : -1.f;
+}
+
+// the block's count of faces that the FP64 solver finished; every thread of the block
+__device__ inline void batch_count(const BatchArgs &a, unsigned long long v,
+                                   unsigned long long *wcount) {
+    if (!a.block_counts) {
+        if (v) atomicAdd(a.fallbacks, v);
         return;
     }
-    if (active) {
-        double rd, ru, rp;
-        int fl;
-        if (precision == MLH_FP64) {
-            GasConst<double> gc(gamma);
-            RSol<double> r = solve_fp64(gc, a0, a1, a2, b0, b1, b2, tol, max_iter, (double)seed, st);
-            rd = r.d; ru = r.u; rp = r.p; fl = r.flag;
-        } else {
-            GasConst<float> gf(gamma);
-            GasConst<double> gc(gamma);
-            RSol<float> r = solve_mixed(gf, gc, (float)a0, (float)a1, (float)a2, (float)b0,
-                                        (float)b1, (float)b2, tol, max_iter, iters32, seed, st);
-            rd = r.d; ru = r.u; rp = r.p; fl = r.flag;
-        }
-        ds[k] = rd; us[k] = ru; ps[k] = rp;
-        if (flag) flag[k] = fl;
-        if (iters) iters[k] = st.iters;
-    }
-    if (!block_counts) {
-        if (st.fallback) atomicAdd(fallbacks, (unsigned long long)st.fallback);
-        return;
-    }
-    // every thread of the block is here: wavefront sums, then the block's
-    unsigned long long v = (unsigned long long)st.fallback;
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
     if ((threadIdx.x & 63) == 0) wcount[threadIdx.x >> 6] = v;
     __syncthreads();
     if (threadIdx.x == 0)
-        block_counts[blockIdx.x] = wcount[0] + wcount[1] + wcount[2] + wcount[3];
+        a.block_counts[blockIdx.x] = wcount[0] + wcount[1] + wcount[2] + wcount[3];
+}
+
+template <int MODE, bool LEARNED>
+__global__ __launch_bounds__(256, !LEARNED && MODE != kSolveMixed ? 3 : 2) void k_riemann_batch(
+    const BatchArgs a) {
+    __shared__ unsigned long long wcount[4];
+    __shared__ uint16_t lds[LEARNED ? 4 : 1][LEARNED ? 64 * 16 : 1];
+    // a wavefront's faces to go on with: list 0 up to iteration kCapSecond,
+    // list 1 to the end.  A list is worked on once it holds 64, so 127 is
+    // the most it reaches.
+    __shared__ double hold_p[4][2][128];
+    __shared__ int hold_at[4][2][128], hold_it[4][2][128];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t base = ((int64_t)blockIdx.x * 4 + wave) * a.tiles * 64;
+    const int64_t rest = a.n - base;
+    const int fresh = rest <= 0 ? 0 : rest < (int64_t)a.tiles * 64 ? (int)rest : a.tiles * 64;
+    unsigned long long fell = 0;
+    int next = 0, held0 = 0, held1 = 0;
+    for (;;) {
+        // a full round of a list first, then new faces, at the end what the
+        // lists still hold
+        int list = -1, m = fresh - next < 64 ? fresh - next : 64;
+        if (held1 >= 64 || (m <= 0 && held0 == 0)) list = 1;
+        else if (held0 >= 64 || m <= 0) list = 0;
+        double s[6] = {1., 0., 1., 1., 0., 1.};
+        SolveHold hold{};
+        int at = next + lane, spent = 0;
+        hold.it = 1;
+        hold.p = -1.0;
+        hold.cap = list < 0 ? kCapFirst : list == 0 ? kCapSecond : a.max_iter;
+        bool active;
+        if (list >= 0) {
+            const int w = list ? held1 : held0;
+            if (w == 0) break;
+            m = w < 64 ? w : 64;
+            active = lane < m;
+            wave_lds_sync();
+            if (active) {
+                at = hold_at[wave][list][w - m + lane];
+                hold.p = hold_p[wave][list][w - m + lane];
+                const int it = hold_it[wave][list][w - m + lane];
+                hold.it = it & 0xff;
+                spent = it >> 8;
+            }
+            wave_lds_sync();
+            if (list) held1 -= m;
+            else held0 -= m;
+        } else {
+            active = lane < m;
+            next += m;
+        }
+        if (active)
+            for (int q = 0; q < 6; ++q) s[q] = a.in[q][base + at];
+        const int64_t k = base + at;
+        const double a0 = s[0], a1 = s[1], a2 = s[2], b0 = s[3], b1 = s[4], b2 = s[5];
+        if (LEARNED && list < 0) {
+            // every lane of the wavefront takes part in the MFMA inference
+            hold.p = (double)batch_seed<4>(a, a0, a1, a2, b0, b1, b2, lds[LEARNED ? wave : 0]);
+        }
+        if (active) {
+            SolveStats st{};
+            st.iters = spent;
+            GasConst<double> gc(a.gamma);
+            RSol<double> r;
+            if (MODE == kSolvePstar) {
+                r.p = star_pressure_fp64<true>(gc, a0, a1, a2, b0, b1, b2, a.tol, a.max_iter, st,
+                                               &hold);
+            } else if (MODE == kSolveMixed && list < 0) {
+                GasConst<float> gf(a.gamma);
+                RSol<float> q = solve_mixed<true>(gf, gc, (float)a0, (float)a1, (float)a2, (float)b0,
+                                                  (float)b1, (float)b2, a.tol, a.max_iter, a.iters32,
+                                                  (float)hold.p, st, &hold);
+                r = RSol<double>{q.d, q.u, q.p, q.flag};
+            } else if (MODE == kSolveMixed) {
+                // the FP32 mode solves the rounded states
+                r = solve_fp64<true>(gc, (float)a0, (float)a1, (float)a2, (float)b0, (float)b1,
+                                     (float)b2, a.tol, a.max_iter, hold.p, st, &hold);
+                r.d = (float)r.d, r.u = (float)r.u, r.p = (float)r.p;
+            } else {
+                r = solve_fp64<true>(gc, a0, a1, a2, b0, b1, b2, a.tol, a.max_iter, hold.p, st,
+                                     &hold);
+            }
+            fell += (unsigned long long)st.fallback;
+            if (!hold.held) {
+                if (MODE == kSolvePstar) {
+                    a.pstar[k] = r.p;
+                } else {
+                    a.ds[k] = r.d, a.us[k] = r.u, a.ps[k] = r.p;
+                    if (a.flag) a.flag[k] = r.flag;
+                }
+                if (a.iters) a.iters[k] = st.iters;
+            }
+            spent = st.iters;
+        }
+        const unsigned long long kept = __ballot(hold.held);
+        const int to = list < 0 ? 0 : 1, held = to ? held1 : held0;
+        if (hold.held) {
+            const int e = held + __popcll(kept & ((1ull << lane) - 1));
+            hold_at[wave][to][e] = at;
+            hold_p[wave][to][e] = hold.p;
+            hold_it[wave][to][e] = spent << 8 | hold.it;
+        }
+        if (to) held1 += __popcll(kept);
+        else held0 += __popcll(kept);
+    }
+    if (MODE != kSolvePstar) batch_count(a, fell, wcount);
+}
+
+// One face per thread, each solved in one go: for batches that give a
+// wavefront of the kernel above no more than a round or two.
+template <int MODE, bool LEARNED>
+__global__ __launch_bounds__(256) void k_riemann_few(const BatchArgs a) {
+    __shared__ unsigned long long wcount[4];
+    __shared__ uint16_t lds[LEARNED ? 4 : 1][LEARNED ? 64 * 16 : 1];
+    const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const bool active = k < a.n;
+    const double a0 = active ? a.in[0][k] : 1., a1 = active ? a.in[1][k] : 0.;
+    const double a2 = active ? a.in[2][k] : 1., b0 = active ? a.in[3][k] : 1.;
+    const double b1 = active ? a.in[4][k] : 0., b2 = active ? a.in[5][k] : 1.;
+    const float seed = LEARNED ? batch_seed<4>(a, a0, a1, a2, b0, b1, b2, lds[threadIdx.x >> 6 & 3]) : -1.f;
+    SolveStats st{};
+    if (active) {
+        GasConst<double> gc(a.gamma);
+        if (MODE == kSolvePstar) {
+            a.pstar[k] = star_pressure_fp64(gc, a0, a1, a2, b0, b1, b2, a.tol, a.max_iter, st);
+        } else {
+            RSol<double> r;
+            if (MODE == kSolveFp64) {
+                r = solve_fp64(gc, a0, a1, a2, b0, b1, b2, a.tol, a.max_iter, (double)seed, st);
+            } else {
+                GasConst<float> gf(a.gamma);
+                RSol<float> q = solve_mixed(gf, gc, (float)a0, (float)a1, (float)a2, (float)b0,
+                                            (float)b1, (float)b2, a.tol, a.max_iter, a.iters32,
+                                            seed, st);
+                r = RSol<double>{q.d, q.u, q.p, q.flag};
+            }
+            a.ds[k] = r.d, a.us[k] = r.u, a.ps[k] = r.p;
+            if (a.flag) a.flag[k] = r.flag;
+        }
+        if (a.iters) a.iters[k] = st.iters;
+    }
+    if (MODE != kSolvePstar) batch_count(a, (unsigned long long)st.fallback, wcount);
+}
+
+// Solves a.n faces on s; the number of blocks.  At most kBatchBlocks (two to
+// three times what is resident at once): a wavefront's lists pay from a few rounds
+// on, and its last ones are part empty.  2^24 states FP64: 1024 blocks 2.33 ms,
+// 1536 2.22, 2048 2.23, 3072 2.34.
+constexpr int kBatchBlocks = 1536;
+// Up to kFewFaces each face in one go: there the lists' rounds come one after the
+// other with nothing beside them.  Random / near-uniform states FP64, in
+// one go against lists: 2^18 241 / 22 us against 275 / 23, 2^19 365 / 36 against
+// 292 / 38, 2^22 2094 / 220 against 720 / 236 (FP32 learned 964 / 343 against
+// 652 / 348).
+constexpr int64_t kFewFaces = 1 << 18;
+template <int MODE, bool LEARNED>
+static int launch_riemann_as(BatchArgs a, hipStream_t s) {
+    const int64_t rounds = (a.n + 255) / 256;
+    if (a.n <= kFewFaces) {
+        hipLaunchKernelGGL((k_riemann_few<MODE, LEARNED>), dim3(rounds), dim3(256), 0, s, a);
+        return (int)rounds;
+    }
+    a.tiles = (int)((rounds + kBatchBlocks - 1) / kBatchBlocks);
+    const int blocks = (int)((rounds + a.tiles - 1) / a.tiles);
+    hipLaunchKernelGGL((k_riemann_batch<MODE, LEARNED>), dim3(blocks), dim3(256), 0, s, a);
+    return blocks;
+}
+static int launch_riemann_batch(BatchArgs a, const double *states, int mode, hipStream_t s) {
+    for (int q = 0; q < 6; ++q) a.in[q] = states + q * a.n;
+    if (mode == kSolvePstar) return launch_riemann_as<kSolvePstar, false>(a, s);
+    if (mode == kSolveFp64)
+        return a.F ? launch_riemann_as<kSolveFp64, true>(a, s)
+                   : launch_riemann_as<kSolveFp64, false>(a, s);
+    return a.F ? launch_riemann_as<kSolveMixed, true>(a, s)
+               : launch_riemann_as<kSolveMixed, false>(a, s);
+}
+
+// the arguments but for the states: outputs and the exact solver's settings
+static BatchArgs batch_args(int64_t n, double gamma, double *star, int *flag, int *iters,
+                            const MlpFrags *F, double tol) {
+    BatchArgs a{};
+    a.n = n, a.gamma = gamma, a.flag = flag, a.iters = iters, a.F = F;
+    a.ds = star, a.us = star + n, a.ps = star + 2 * n;
+    a.tol = tol, a.max_iter = 50, a.iters32 = 3;
+    return a;
 }
 
 // out[0] = sum of in[0..n) (one block of 256 threads)
@@ -1038,11 +1220,9 @@ int mlh_riemann_exact_batch(mlh_ctx *c, int64_t n, double gamma, const double *r
     const double *in[6] = {rhoL, uL, PL, rhoR, uR, PR};
     for (int k = 0; k < 6; ++k) hipMemcpyAsync(buf + k * n, in[k], b, hipMemcpyHostToDevice, s);
     hipMemsetAsync(fb, 0, sizeof(unsigned long long), s);
-    int max_iter = 50;
-    hipLaunchKernelGGL(k_riemann_batch, dim3((n + 255) / 256), dim3(256), 0, s, n, gamma, buf,
-                       buf + n, buf + 2 * n, buf + 3 * n, buf + 4 * n, buf + 5 * n, buf + 6 * n,
-                       buf + 7 * n, buf + 8 * n, ib, ib + n, precision, F, tol, max_iter, 3, fb,
-                       nullptr, nullptr);
+    BatchArgs a = batch_args(n, gamma, buf + 6 * n, ib, ib + n, F, tol);
+    a.fallbacks = fb;
+    launch_riemann_batch(a, buf, precision == MLH_FP64 ? kSolveFp64 : kSolveMixed, s);
     hipMemcpyAsync(rho_s, buf + 6 * n, b, hipMemcpyDeviceToHost, s);
     hipMemcpyAsync(u_s, buf + 7 * n, b, hipMemcpyDeviceToHost, s);
     hipMemcpyAsync(P_s, buf + 8 * n, b, hipMemcpyDeviceToHost, s);
@@ -1103,10 +1283,9 @@ int mlh_riemann_exact_batch_device(mlh_ctx *c, int64_t n, double gamma, const do
     hipEventCreate(&e1);
     hipMemsetAsync(fb, 0, sizeof(unsigned long long), s);
     hipEventRecord(e0, s);
-    hipLaunchKernelGGL(k_riemann_batch, dim3((n + 255) / 256), dim3(256), 0, s, n, gamma, states,
-                       states + n, states + 2 * n, states + 3 * n, states + 4 * n, states + 5 * n,
-                       star, star + n, star + 2 * n, flag, iters, precision, F, tol, 50, 3, fb,
-                       nullptr, nullptr);
+    BatchArgs a = batch_args(n, gamma, star, flag, iters, F, tol);
+    a.fallbacks = fb;
+    launch_riemann_batch(a, states, precision == MLH_FP64 ? kSolveFp64 : kSolveMixed, s);
     hipEventRecord(e1, s);
     unsigned long long h_fb = 0;
     hipMemcpyAsync(&h_fb, fb, sizeof(h_fb), hipMemcpyDeviceToHost, s);
@@ -1178,11 +1357,10 @@ int mlh_riemann_exact_batch_device_noalloc(mlh_ctx *c, int64_t n, double gamma,
     int st = batch_scratch(&scr);
     if (st) return st;
     hipStream_t s = c ? ctx_stream(c) : nullptr;
-    const int nblocks = (int)((n + 255) / 256);  // <= kNoAllocBlocks
-    hipLaunchKernelGGL(k_riemann_batch, dim3(nblocks), dim3(256), 0, s, n, gamma, states,
-                       states + n, states + 2 * n, states + 3 * n, states + 4 * n, states + 5 * n,
-                       star, star + n, star + 2 * n, flag, iters, precision, F, tol, 50, 3,
-                       nullptr, nullptr, scr);
+    BatchArgs a = batch_args(n, gamma, star, flag, iters, F, tol);
+    a.block_counts = scr;
+    const int nblocks =  // <= kNoAllocBlocks
+        launch_riemann_batch(a, states, precision == MLH_FP64 ? kSolveFp64 : kSolveMixed, s);
     hipLaunchKernelGGL(k_sum_u64, dim3(1), dim3(256), 0, s, scr, nblocks, scr + kNoAllocBlocks);
     unsigned long long total = 0;
     CHK(hipMemcpyAsync(&total, scr + kNoAllocBlocks, sizeof(total), hipMemcpyDeviceToHost, s));
@@ -1207,9 +1385,9 @@ int mlh_riemann_pstar_batch(int64_t n, double gamma, const double *rhoL, const d
     size_t b = sizeof(double) * n;
     const double *in[6] = {rhoL, uL, PL, rhoR, uR, PR};
     for (int k = 0; k < 6; ++k) hipMemcpy(buf + k * n, in[k], b, hipMemcpyHostToDevice);
-    hipLaunchKernelGGL(k_riemann_batch, dim3((n + 255) / 256), dim3(256), 0, 0, n, gamma, buf,
-                       buf + n, buf + 2 * n, buf + 3 * n, buf + 4 * n, buf + 5 * n, buf, buf, buf,
-                       nullptr, ib, MLH_FP64, nullptr, tol, 50, 3, fb, buf + 6 * n, nullptr);
+    BatchArgs a = batch_args(n, gamma, buf, nullptr, ib, nullptr, tol);
+    a.pstar = buf + 6 * n;
+    launch_riemann_batch(a, buf, kSolvePstar, 0);
     hipMemcpy(p_star, buf + 6 * n, b, hipMemcpyDeviceToHost);
     if (iters) hipMemcpy(iters, ib, sizeof(int) * n, hipMemcpyDeviceToHost);
     hipError_t e = hipDeviceSynchronize();

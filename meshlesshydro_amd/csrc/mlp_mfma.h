@@ -119,12 +119,13 @@ __device__ inline float mlp_infer_wave_bf16_mem(const MlpFrags *__restrict__ F, 
     return mlp_infer_wave_bf16(R, x, lds);
 }
 
-// Register-lean variant for the face kernel: one face tile (16 faces) at a
-// time, layer 1 straight into the packed BF16 operand of layer 2 (the lane
+// Register-lean variant for the face kernel: U face tiles (16 faces each) at
+// a time, layer 1 straight into the packed BF16 operand of layer 2 (the lane
 // that computes neurons 4g..4g+3 of face c is the lane that needs them), and
-// each weight fragment read from memory (L1 resident) where it is used.
-// About 30 VGPRs live instead of ~170; the arithmetic is that of
-// mlp_infer_wave_bf16 except for the order of the output-layer sums.
+// each weight fragment read from memory (L1 resident) where it is used, once
+// per U tiles.  About 30 VGPRs live (U = 1) instead of ~170; the arithmetic
+// is that of mlp_infer_wave_bf16.
+template <int U = 1>
 __device__ inline float mlp_infer_wave_bf16_lean(const MlpFrags *__restrict__ F,
                                                  const float *x, uint16_t *lds) {
     const int l = __lane_id(), g = l >> 4, c = l & 15;
@@ -140,42 +141,56 @@ __device__ inline float mlp_infer_wave_bf16_lean(const MlpFrags *__restrict__ F,
     wave_lds_sync();
     float out = 0.f;
 #pragma unroll 1
-    for (int nt = 0; nt < 4; ++nt) {
+    for (int n0 = 0; n0 < 4; n0 += U) {
         // keeps the fragment loads inside the loop (no hoisting into registers)
         asm volatile("" ::: "memory");
-        bf16x8_t bx;
-        if (g < 2) {
-            bx = *(const bf16x8_t *)&lds[(16 * nt + c) * 16 + 8 * g];
-        } else {
-            for (int j = 0; j < 8; ++j) bx[j] = (__bf16)0.f;
+        bf16x8_t bx[U], b0[U], b1[U];
+        f32x4_t p[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (g < 2) {
+                bx[u] = *(const bf16x8_t *)&lds[(16 * (n0 + u) + c) * 16 + 8 * g];
+            } else {
+                for (int j = 0; j < 8; ++j) bx[u][j] = (__bf16)0.f;
+            }
+            p[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         }
-        bf16x8_t b0, b1;
+#pragma unroll
         for (int mt = 0; mt < 4; ++mt) {
             bf16x8_t w = *(const bf16x8_t *)&F->w1[mt][l][0];
             f32x4_t bias = *(const f32x4_t *)&F->b1[mt][l][0];
-            f32x4_t acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, bx, bias, 0, 0, 0);
-            for (int r = 0; r < 4; ++r) {
-                __bf16 h = (__bf16)tanh_fast(acc[r]);
-                if (mt == 0) b0[r] = h;
-                else if (mt == 1) b0[4 + r] = h;
-                else if (mt == 2) b1[r] = h;
-                else b1[4 + r] = h;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                f32x4_t acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, bx[u], bias, 0, 0, 0);
+                for (int r = 0; r < 4; ++r) {
+                    __bf16 h = (__bf16)tanh_fast(acc[r]);
+                    if (mt == 0) b0[u][r] = h;
+                    else if (mt == 1) b0[u][4 + r] = h;
+                    else if (mt == 2) b1[u][r] = h;
+                    else b1[u][4 + r] = h;
+                }
             }
         }
-        f32x4_t p = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
         for (int mo = 0; mo < 4; ++mo) {
             bf16x8_t wa = *(const bf16x8_t *)&F->w2[mo][0][l][0];
             bf16x8_t wb = *(const bf16x8_t *)&F->w2[mo][1][l][0];
             f32x4_t bias = *(const f32x4_t *)&F->b2[mo][l][0];
             f32x4_t w3 = *(const f32x4_t *)&F->w3[mo][l][0];
-            f32x4_t acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, b0, bias, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb, b1, acc, 0, 0, 0);
-            for (int r = 0; r < 4; ++r) p[r] += w3[r] * tanh_fast(acc[r]);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                f32x4_t acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, b0[u], bias, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb, b1[u], acc, 0, 0, 0);
+                for (int r = 0; r < 4; ++r) p[u][r] += w3[r] * tanh_fast(acc[r]);
+            }
         }
-        float v = p[0] + p[1] + p[2] + p[3];
-        v += __shfl_xor(v, 16, 64);
-        v += __shfl_xor(v, 32, 64);
-        if (g == nt) out = v;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            float v = p[u][0] + p[u][1] + p[u][2] + p[u][3];
+            v += __shfl_xor(v, 16, 64);
+            v += __shfl_xor(v, 32, 64);
+            if (g == n0 + u) out = v;
+        }
     }
     return out + F->b3;
 }

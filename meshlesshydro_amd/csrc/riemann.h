@@ -303,12 +303,24 @@ struct SolveStats {
     int acoustic;   // FP32: near-uniform faces given the acoustic solution
 };
 
+// A solve that may stop early, for a caller that gathers the faces which need
+// longer and goes on with them together: FP64 Newton stops after iteration
+// `cap` (mixed solves: before any FP64 iteration), with `held` set and what it
+// needs to go on.  The same bits come out as from a solve in one go.
+struct SolveHold {
+    int cap;      // last iteration of this part (>= max_iter: to the end)
+    int it;       // next iteration (1: from the start, p as p0)
+    double p;     // its iterate
+    bool held;    // stopped early: no solution yet
+};
+
 // Plain FP64 exact solver from the standard guess (or from p0 > 0).
+template <bool kHold = false>
 __device__ inline RSol<double> solve_fp64(const GasConst<double> &c, double dl,
                                           double ul, double pl, double dr,
                                           double ur, double pr, double tol,
                                           int max_iter, double p0,
-                                          SolveStats &st) {
+                                          SolveStats &st, SolveHold *hold = nullptr) {
     if (!(dl > 0.0) || !(dr > 0.0)) {
         double cl = dl > 0.0 ? sqrt(c.g * pl / dl) : 0.0;
         double cr = dr > 0.0 ? sqrt(c.g * pr / dr) : 0.0;
@@ -320,8 +332,15 @@ __device__ inline RSol<double> solve_fp64(const GasConst<double> &c, double dl,
     double tiny = tol * 0.5 * (pl + pr);
     double pold = p0 > 0.0 ? p0 : guess_p(c, dl, ul, pl, cl, dr, ur, pr, cr, tiny);
     double p = pold, fl, fld, fr, frd;
-    int it;
-    for (it = 1; it <= max_iter; ++it) {
+    int it = 1, last = max_iter;
+    if (kHold) {
+        if (hold->it > 1) {
+            it = hold->it;
+            pold = hold->p;
+        }
+        if (hold->cap < last) last = hold->cap;
+    }
+    for (; it <= last; ++it) {
         prefun(c, pold, dl, pl, cl, fl, fld);
         prefun(c, pold, dr, pr, cr, fr, frd);
         p = pold - (fl + fr + du) / (fld + frd);
@@ -329,6 +348,12 @@ __device__ inline RSol<double> solve_fp64(const GasConst<double> &c, double dl,
         if (change <= tol) break;
         if (p < 0.0) p = tiny;
         pold = p;
+    }
+    if (kHold && it > last && last < max_iter) {
+        hold->it = it;
+        hold->p = pold;
+        hold->held = true;
+        return RSol<double>{0., 0., 0., 0};
     }
     if (it > max_iter) {
         st.nonconv += 1;
@@ -344,9 +369,11 @@ __device__ inline RSol<double> solve_fp64(const GasConst<double> &c, double dl,
 }
 
 // Converged star pressure p* of the plain FP64 solver (0 for vacuum).
+template <bool kHold = false>
 __device__ inline double star_pressure_fp64(const GasConst<double> &c, double dl, double ul,
                                             double pl, double dr, double ur, double pr,
-                                            double tol, int max_iter, SolveStats &st) {
+                                            double tol, int max_iter, SolveStats &st,
+                                            SolveHold *hold = nullptr) {
     if (!(dl > 0.0) || !(dr > 0.0)) return 0.0;
     double cl = sqrt(c.g * pl / dl), cr = sqrt(c.g * pr / dr);
     double du = ur - ul;
@@ -354,8 +381,15 @@ __device__ inline double star_pressure_fp64(const GasConst<double> &c, double dl
     double tiny = tol * 0.5 * (pl + pr);
     double pold = guess_p(c, dl, ul, pl, cl, dr, ur, pr, cr, tiny);
     double p = pold, fl, fld, fr, frd;
-    int it;
-    for (it = 1; it <= max_iter; ++it) {
+    int it = 1, last = max_iter;
+    if (kHold) {
+        if (hold->it > 1) {
+            it = hold->it;
+            pold = hold->p;
+        }
+        if (hold->cap < last) last = hold->cap;
+    }
+    for (; it <= last; ++it) {
         prefun(c, pold, dl, pl, cl, fl, fld);
         prefun(c, pold, dr, pr, cr, fr, frd);
         p = pold - (fl + fr + du) / (fld + frd);
@@ -363,6 +397,12 @@ __device__ inline double star_pressure_fp64(const GasConst<double> &c, double dl
         if (change <= tol) break;
         if (p < 0.0) p = tiny;
         pold = p;
+    }
+    if (kHold && it > last && last < max_iter) {
+        hold->it = it;
+        hold->p = pold;
+        hold->held = true;
+        return 0.0;
     }
     if (it > max_iter) {
         int nb = 0;
@@ -455,10 +495,12 @@ __device__ inline MixedProbe mixed_probe(const GasConst<float> &cf, const GasCon
     return m;
 }
 
+template <bool kHold = false>
 __device__ inline RSol<float> mixed_finish(const GasConst<float> &cf, const GasConst<double> &cd,
                                            float dl, float ul, float pl, float dr, float ur,
                                            float pr, double tol, int max_iter, int iters32,
-                                           float restart, const MixedProbe &m, SolveStats &st) {
+                                           float restart, const MixedProbe &m, SolveStats &st,
+                                           SolveHold *hold = nullptr) {
     if (m.acoustic) {
         // the star state on the contact's upwind side (x/t = 0 lies between
         // the acoustic waves)
@@ -499,20 +541,29 @@ __device__ inline RSol<float> mixed_finish(const GasConst<float> &cf, const GasC
     // FP64 fallback, from the last FP64 step when it is positive (the FP32
     // root refined once: far closer than the standard guess), else from the
     // standard guess
-    RSol<double> r = solve_fp64(cd, dl, ul, pl, dr, ur, pr, tol, max_iter,
-                                m.valid && pn > 0.0 ? pn : -1.0, st);
+    const double p0 = m.valid && pn > 0.0 ? pn : -1.0;
+    if (kHold) {
+        hold->it = 1;
+        hold->p = p0;
+        hold->held = true;
+        return RSol<float>{0.f, 0.f, 0.f, 0};
+    }
+    RSol<double> r = solve_fp64(cd, dl, ul, pl, dr, ur, pr, tol, max_iter, p0, st);
     return RSol<float>{float(r.d), float(r.u), float(r.p), r.flag};
 }
 
 // probe at p_seed (the standard guess when <= 0), then finish
+template <bool kHold = false>
 __device__ inline RSol<float> solve_mixed(const GasConst<float> &cf,
                                           const GasConst<double> &cd, float dl,
                                           float ul, float pl, float dr,
                                           float ur, float pr, double tol,
                                           int max_iter, int iters32,
-                                          float p_seed, SolveStats &st) {
+                                          float p_seed, SolveStats &st,
+                                          SolveHold *hold = nullptr) {
     MixedProbe m = mixed_probe(cf, cd, dl, ul, pl, dr, ur, pr, tol, p_seed, st);
-    return mixed_finish(cf, cd, dl, ul, pl, dr, ur, pr, tol, max_iter, iters32, -1.f, m, st);
+    return mixed_finish<kHold>(cf, cd, dl, ul, pl, dr, ur, pr, tol, max_iter, iters32, -1.f, m, st,
+                               hold);
 }
 
 }  // namespace mlh
