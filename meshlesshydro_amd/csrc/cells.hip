@@ -485,6 +485,44 @@ __device__ inline uint32_t stage_word(uint32_t jo, const int *s) {
     return (jo << 6) | ((7u - m) << 3) | sg;
 }
 
+// staged sort word -> row entry (index | code)
+template <bool kCaller>
+__device__ inline uint32_t row_entry(const NbrArgs &a, uint32_t w) {
+    const uint32_t jo = w >> 6, m = 7u - ((w >> 3) & 7u);
+    uint32_t code = 0, mul = 1;
+    for (int ax = 0; ax < 3; ++ax, mul *= 3)
+        code += mul * (((m >> ax) & 1u) ? (((w >> ax) & 1u) ? 2u : 0u) : 1u);
+    return (kCaller ? jo : a.inv[jo]) | (code << kIdxBits);
+}
+
+// virtual cell v: shifts s and the real cell r; whether any axis wraps
+template <int D>
+__device__ inline bool wrapped_cell(const Geom &g, const int *v, int *s, int *r) {
+    bool wrapped = false;
+    for (int ax = 0; ax < D; ++ax) {
+        s[ax] = v[ax] < 0 ? -1 : (v[ax] >= g.nc[ax] ? 1 : 0);
+        r[ax] = v[ax] - s[ax] * g.nc[ax];
+        wrapped |= s[ax] != 0;
+    }
+    return wrapped;
+}
+
+// the reference's ghost creation test of parent pj for shifts s, and the
+// distance test of the image
+template <int D>
+__device__ inline bool is_image(const Geom &g, const int *s, const double4 &pj, const double *xi) {
+    double xj[3] = {pj.x, pj.y, pj.z};
+    bool exists = true;
+    for (int ax = 0; ax < D; ++ax) {
+        if (s[ax] == 0) continue;
+        bool low = xj[ax] <= g.bmin[ax] + g.h;
+        bool high = g.bmax[ax] - g.h < xj[ax];
+        exists &= s[ax] > 0 ? low : (!low && high);
+        xj[ax] = image_coord(xj[ax], s[ax], g.bmin[ax], g.bmax[ax]);
+    }
+    return exists && dist2<D>(xj, xi) < g.hsq;
+}
+
 // Periodic images of work position t (position xi, cell cc) in the
 // reference's ghost order, stored in its row from entry g0 on: only
 // particles whose cell lies within the image window of a domain face
@@ -508,14 +546,7 @@ __device__ inline int image_search(const NbrArgs &a, int t, const double *xi, co
     for (int ax = 0; ax < D; ++ax) near_edge |= cc[ax] - W < 0 || cc[ax] + W >= g.nc[ax];
     if (g.periodic && near_edge) {
         uint32_t *nb = a.nbr;
-        // staged sort word -> row entry (index | code)
-        auto to_row = [&](uint32_t w) {
-            const uint32_t jo = w >> 6, m = 7u - ((w >> 3) & 7u);
-            uint32_t code = 0, mul = 1;
-            for (int ax = 0; ax < 3; ++ax, mul *= 3)
-                code += mul * (((m >> ax) & 1u) ? (((w >> ax) & 1u) ? 2u : 0u) : 1u);
-            return (kCaller ? jo : a.inv[jo]) | (code << kIdxBits);
-        };
+        auto to_row = [&](uint32_t w) { return row_entry<kCaller>(a, w); };
         // entries are in the row: the stage overflowed, or parents are too
         // large for sort words
         bool in_row = (uint32_t)N > (1u << kStageIdxBits);
@@ -524,31 +555,14 @@ __device__ inline int image_search(const NbrArgs &a, int t, const double *xi, co
                 for (int vx = cc[0] - W; vx <= cc[0] + W && !err; ++vx) {
                     int v[3] = {vx, vy, vz};
                     int s[3] = {0, 0, 0}, r[3] = {0, 0, 0};
-                    bool wrapped = false;
-                    for (int ax = 0; ax < D; ++ax) {
-                        s[ax] = v[ax] < 0 ? -1 : (v[ax] >= g.nc[ax] ? 1 : 0);
-                        r[ax] = v[ax] - s[ax] * g.nc[ax];
-                        wrapped |= s[ax] != 0;
-                    }
-                    if (!wrapped) continue;
+                    if (!wrapped_cell<D>(g, v, s, r)) continue;
                     uint32_t c = cell_key<D>(g, r[0], r[1], r[2]);
                     uint32_t code = (uint32_t)((s[0] + 1) + 3 * (s[1] + 1) + 9 * (s[2] + 1));
                     const uint32_t cw = stage_word(0, s);
                     // one candidate: the reference's ghost creation test and
                     // image, the distance test, the entry in ghost order
                     auto visit = [&](int q, const double4 &pj) {
-                        double xj[3] = {pj.x, pj.y, pj.z};
-                        bool exists = true;
-                        for (int ax = 0; ax < D; ++ax) {
-                            if (s[ax] == 0) continue;
-                            bool low = xj[ax] <= g.bmin[ax] + g.h;
-                            bool high = g.bmax[ax] - g.h < xj[ax];
-                            exists &= s[ax] > 0 ? low : (!low && high);
-                            xj[ax] = image_coord(xj[ax], s[ax], g.bmin[ax], g.bmax[ax]);
-                        }
-                        if (!exists) return;
-                        double d = dist2<D>(xj, xi);
-                        if (!(d < g.hsq)) return;
+                        if (!is_image<D>(g, s, pj, xi)) return;
                         if (gcnt >= a.maxg) {
                             err = 1;
                             return;
@@ -790,23 +804,87 @@ __device__ inline uint32_t face_slots(unsigned long long *nfaces, int own) {
 // The periodic image search, on a stream of its own beside k_neighbours: a
 // particle whose cell lies within the image window of a domain face stores
 // its images from row entry img_base on (behind every sector the real
-// search stores) and their count in img_cnt.  One thread per work position
-// (cell order: a wavefront's particles lie near the same domain faces), one
-// wavefront per block; a lane's kImgStage LDS slots are interleaved with
-// its neighbours' (slot k of lane l at k * 64 + l: no bank conflicts).
-constexpr int kImgThreads = 64;
+// search stores) and their count in img_cnt.
+// A wavefront looks at `per` work positions and searches those with images
+// eight at a time, kImgLanes lanes to a particle: each lane takes every eighth
+// cell of the window and appends its hits to the particle's LDS stage in any
+// order; the sort words are distinct, so a hit's place in the row is the number
+// of smaller words.  A particle whose images do not fit the stage, the capacity
+// or the words goes through image_search on one lane.
+// A wavefront's time is its particles' dependent loads, not the work: one
+// particle per lane 97 us at 32^2, 594 at 24^3, 206 at 1000^2; here 27, 122, 167
+// (turbulence 160^3 with `per` 64 1391 -> 1041; blast 128^3 589 -> 663, beside
+// 1600 us of k_neighbours).
+// images a particle's group holds (turbulence with 64 neighbours: 64 at a corner)
+constexpr int kImgThreads = 64, kImgLanes = 8, kImgGroups = kImgThreads / kImgLanes;
+constexpr int kGroupStage = 128;
+static_assert(kGroupStage >= kImgStage, "image_search sorts in a group's stage");
 template <int D, bool kCaller>
-__global__ __launch_bounds__(kImgThreads) void k_images(NbrArgs a) {
-    __shared__ uint32_t s_stage[kImgThreads * kImgStage];
-    const int t = xcd_block() * blockDim.x + threadIdx.x;
-    if (t >= a.N) return;
+__global__ __launch_bounds__(kImgThreads) void k_images(NbrArgs a, int per) {
+    __shared__ uint32_t s_stage[kImgGroups][kGroupStage + 1];
+    __shared__ uint32_t s_list[kImgThreads];
+    __shared__ uint32_t s_n[kImgGroups];
+    const int lane = threadIdx.x, grp = lane / kImgLanes, l = lane % kImgLanes;
+    const int t0 = xcd_block() * per + lane;
     int cc[3];
-    cell_coords<D>(a.g, a.ck_w[t], cc);
-    if (!has_images<D>(a, cc)) return;
-    const double4 pi = a.pos_w[t];
-    const double xi[3] = {pi.x, pi.y, pi.z};
-    a.img_cnt[t] = image_search<D, kCaller>(a, t, xi, cc, a.img_base, s_stage + threadIdx.x,
-                                            kImgThreads);
+    bool mine = lane < per && t0 < a.N;
+    if (mine) {
+        cell_coords<D>(a.g, a.ck_w[t0], cc);
+        mine = has_images<D>(a, cc);
+    }
+    const unsigned long long m = __ballot(mine);
+    if (mine) s_list[__popcll(m & ((1ull << lane) - 1))] = (uint32_t)t0;
+    wave_lds_sync();
+    const int todo = __popcll(m);
+    const Geom &g = a.g;
+    const int W = a.img_window, side = 2 * W + 1, ncell = D == 3 ? side * side * side : side * side;
+    for (int b = 0; b < todo; b += kImgGroups) {
+        const bool on = b + grp < todo;
+        const int t = (int)s_list[on ? b + grp : b];
+        if (l == 0) s_n[grp] = 0;
+        wave_lds_sync();
+        cell_coords<D>(g, a.ck_w[t], cc);
+        const double4 pi = a.pos_w[t];
+        const double xi[3] = {pi.x, pi.y, pi.z};
+        for (int c = l; on && c < ncell; c += kImgLanes) {
+            const int cy = c / side;
+            int v[3] = {cc[0] - W + c % side, cc[1] - W + (D == 3 ? cy % side : cy),
+                        D == 3 ? cc[2] - W + cy / side : 0};
+            int s[3] = {0, 0, 0}, r[3] = {0, 0, 0};
+            if (!wrapped_cell<D>(g, v, s, r)) continue;
+            const uint32_t key = cell_key<D>(g, r[0], r[1], r[2]), cw = stage_word(0, s);
+            const int q0 = a.cstart[key], q1 = a.cend[key];
+            for (int q = q0; q < q1; q += 4) {
+                double4 pb[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) pb[u] = a.pos_cell[q + u < q1 ? q + u : q1 - 1];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (q + u < q1 && is_image<D>(g, s, pb[u], xi)) {
+                        const uint32_t k = atomicAdd(&s_n[grp], 1u);
+                        if (k < (uint32_t)kGroupStage)
+                            s_stage[grp][k] = ((uint32_t)pb[u].w << 6) | cw;
+                    }
+            }
+        }
+        wave_lds_sync();
+        const int n = (int)s_n[grp];
+        if (on) {
+            if (n > kGroupStage || n > a.maxg || (uint32_t)a.N > (1u << kStageIdxBits)) {
+                if (l == 0)
+                    a.img_cnt[t] = image_search<D, kCaller>(a, t, xi, cc, a.img_base, s_stage[grp], 1);
+            } else {
+                for (int e = l; e < n; e += kImgLanes) {
+                    const uint32_t w = s_stage[grp][e];
+                    int rank = 0;
+                    for (int k = 0; k < n; ++k) rank += s_stage[grp][k] < w;
+                    a.nbr[nb_slot(a.N, t, a.img_base + rank)] = row_entry<kCaller>(a, w);
+                }
+                if (l == 0) a.img_cnt[t] = n;
+            }
+        }
+        wave_lds_sync();
+    }
 }
 
 // After k_neighbours and k_images: for the particles k_neighbours left their
@@ -1097,6 +1175,11 @@ void launch_pack_pos(const double *x0, const double *x1, const double *x2, int D
     hipLaunchKernelGGL(k_pack_pos, dim3((N + 255) / 256), dim3(256), 0, s, x0, x1, x2, D, N, pos);
 }
 
+// Work positions a wavefront of k_images looks at: eight while that gives
+// wavefronts for the whole chip only, then 64, since most find no particle
+// with images (8 against 64: blast 64^3 212 / 326 us, shear 1000^2 167 / 276,
+// turbulence 160^3 1263 / 1041, blast 128^3 684 / 663).
+constexpr int kImgSpread = 1 << 20;
 struct NbrStreams {
     hipStream_t s, s_img;
     hipEvent_t fork, join;
@@ -1109,8 +1192,9 @@ static void launch_nbr_dens(const NbrArgs &a, dim3 grid, const NbrStreams &st) {
     if (a.g.periodic) {
         hipEventRecord(st.fork, st.s);
         hipStreamWaitEvent(st.s_img, st.fork, 0);
-        hipLaunchKernelGGL((k_images<D, kCaller>), dim3((a.N + kImgThreads - 1) / kImgThreads),
-                           dim3(kImgThreads), 0, st.s_img, a);
+        const int per = a.N <= kImgSpread ? kImgGroups : kImgThreads;
+        hipLaunchKernelGGL((k_images<D, kCaller>), dim3((a.N + per - 1) / per), dim3(kImgThreads),
+                           0, st.s_img, a, per);
         hipEventRecord(st.join, st.s_img);
     }
     hipLaunchKernelGGL((k_neighbours<D, kCaller, kDens>), grid, dim3(256), 0, st.s, a);
