@@ -41,11 +41,6 @@
 
 namespace mlh {
 
-__global__ void k_fill_i32(int *p, int v, int n) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) p[t] = v;
-}
-
 // key of the cell of (x0, x1, x2)
 template <int D>
 __device__ inline uint32_t key_of(const Geom &g, double x0, double x1, double x2) {
@@ -64,24 +59,29 @@ template <int D>
 __global__ void k_assign_cells(Geom g, const double *__restrict__ x0,
                                const double *__restrict__ x1,
                                const double *__restrict__ x2, int N,
-                               uint32_t *__restrict__ key, uint32_t *__restrict__ idx,
-                               unsigned long long *__restrict__ nfaces) {
+                               uint32_t *__restrict__ key, int *__restrict__ cstart,
+                               int *__restrict__ cend, unsigned long long *__restrict__ nfaces) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i == 0) *nfaces = 0;  // the search's face slots
+    // every cell empty
+    for (int c = i; c < g.nkeys; c += gridDim.x * blockDim.x) cstart[c] = cend[c] = 0;
     if (i >= N) return;
     key[i] = key_of<D>(g, x0[i], x1[i], D == 3 ? x2[i] : 0.0);
-    idx[i] = (uint32_t)i;
 }
 
 // positions in cell order; w = original index (exact in a double); inv:
-// original index -> cell-order position
+// original index -> cell-order position; the cells' ranges of positions
 __global__ void k_gather_pos(const double *__restrict__ x0, const double *__restrict__ x1,
                              const double *__restrict__ x2, int D, int N,
-                             const uint32_t *__restrict__ sidx, double4 *__restrict__ pos,
-                             uint32_t *__restrict__ inv) {
+                             const uint32_t *__restrict__ skeys, const uint32_t *__restrict__ sidx,
+                             double4 *__restrict__ pos, uint32_t *__restrict__ inv,
+                             int *__restrict__ cstart, int *__restrict__ cend) {
     int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= N) return;
     uint32_t i = sidx[t];
+    const uint32_t k = skeys[t];
+    if (t == 0 || skeys[t - 1] != k) cstart[k] = t;
+    if (t == N - 1 || skeys[t + 1] != k) cend[k] = t + 1;
     pos[t] = make_double4(x0[i], x1[i], D == 3 ? x2[i] : 0.0, (double)i);
     inv[i] = (uint32_t)t;
 }
@@ -135,7 +135,7 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(
         int e = base + r * kRsThreads + tid;
         bool valid = e < N;
         uint32_t k = valid ? kin[e] : 0u;
-        uint32_t v = valid ? vin[e] : 0u;
+        uint32_t v = vin ? (valid ? vin[e] : 0u) : (uint32_t)e;
         uint32_t d = (k >> shift) & mask;
         uint64_t m = __ballot(valid);
         for (int b = 0; b < dbits; ++b) {
@@ -238,6 +238,30 @@ size_t radix_sort_scratch_words(int N) {
     return 2 * h + (h + kScanBlock - 1) / kScanBlock + 16;
 }
 
+// Stable sort of keys `kin` (left as they are) with their places as values, by
+// the low `bits` bits: result in (k0, v0); (k1, v1) is ping-pong space.  The
+// first pass reads kin and counts places itself, the last one lands in (k0, v0).
+static void radix_sort_places(const uint32_t *kin, uint32_t *k0, uint32_t *v0, uint32_t *k1,
+                              uint32_t *v1, int N, int bits, uint32_t *scratch, hipStream_t s) {
+    int ntiles = (N + kRsTile - 1) / kRsTile;
+    const int passes = (bits + kRsMaxBits - 1) / kRsMaxBits;
+    const int dbits = (bits + passes - 1) / passes;
+    uint32_t *hist = scratch, *offs = scratch + (size_t)kRsMaxBins * ntiles,
+             *tmp = scratch + 2 * (size_t)kRsMaxBins * ntiles;
+    const uint32_t *vin = nullptr;
+    for (int p = 0; p < passes; ++p) {
+        const bool to0 = (passes - 1 - p) % 2 == 0;
+        uint32_t *ko = to0 ? k0 : k1, *vo = to0 ? v0 : v1;
+        hipLaunchKernelGGL(k_rs_hist, dim3(ntiles), dim3(kRsThreads), 0, s, kin, N, dbits * p, dbits,
+                           hist, ntiles);
+        scan_exclusive_u32(hist, offs, (1 << dbits) * ntiles, tmp, s);
+        hipLaunchKernelGGL(k_rs_scatter, dim3(ntiles), dim3(kRsThreads), 0, s, kin, vin, ko, vo, N,
+                           dbits * p, dbits, offs, ntiles);
+        kin = ko;
+        vin = vo;
+    }
+}
+
 // Stable sort of (key, val) by the low `bits` bits of key.  Result in
 // (k0, v0); (k1, v1) is ping-pong space.
 void radix_sort_pairs(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, int N,
@@ -263,15 +287,6 @@ void radix_sort_pairs(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, in
         hipMemcpyAsync(k1, k0, sizeof(uint32_t) * N, hipMemcpyDeviceToDevice, s);
         hipMemcpyAsync(v1, v0, sizeof(uint32_t) * N, hipMemcpyDeviceToDevice, s);
     }
-}
-
-__global__ void k_cell_ranges(const uint32_t *__restrict__ skeys, int N,
-                              int *__restrict__ cstart, int *__restrict__ cend) {
-    int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= N) return;
-    uint32_t k = skeys[p];
-    if (p == 0 || skeys[p - 1] != k) cstart[k] = p;
-    if (p == N - 1 || skeys[p + 1] != k) cend[k] = p + 1;
 }
 
 // The whole cell list of a small problem in one block: keys, stable sort, cell
@@ -978,9 +993,9 @@ __global__ __launch_bounds__(256) void k_neighbours(NbrArgs a) {
 }
 
 template __global__ void k_assign_cells<2>(Geom, const double *, const double *, const double *,
-                                           int, uint32_t *, uint32_t *, unsigned long long *);
+                                           int, uint32_t *, int *, int *, unsigned long long *);
 template __global__ void k_assign_cells<3>(Geom, const double *, const double *, const double *,
-                                           int, uint32_t *, uint32_t *, unsigned long long *);
+                                           int, uint32_t *, int *, int *, unsigned long long *);
 // ------------------------------------------------------------ domain limits
 // Particles::getDomainLimits (Particles.cpp:228-268) as the reference runs
 // it, sequentially per axis: min starts at DBL_MAX, max at DBL_MIN (the
@@ -1156,18 +1171,15 @@ void launch_cells(const Geom &g, int D, const double *x0, const double *x1,
         return;
     }
     if (D == 2)
-        hipLaunchKernelGGL(k_assign_cells<2>, dim3(nb), dim3(256), 0, s, g, x0, x1, x2, N, key, idx, nfaces);
+        hipLaunchKernelGGL(k_assign_cells<2>, dim3(nb), dim3(256), 0, s, g, x0, x1, x2, N, key, cstart,
+                           cend, nfaces);
     else
-        hipLaunchKernelGGL(k_assign_cells<3>, dim3(nb), dim3(256), 0, s, g, x0, x1, x2, N, key, idx, nfaces);
-    // sort a copy: key[i] stays the cell of particle i
-    hipMemcpyAsync(skey, key, sizeof(uint32_t) * N, hipMemcpyDeviceToDevice, s);
+        hipLaunchKernelGGL(k_assign_cells<3>, dim3(nb), dim3(256), 0, s, g, x0, x1, x2, N, key, cstart,
+                           cend, nfaces);
     uint32_t *k1 = scratch, *v1 = scratch + N, *rs = scratch + 2 * (size_t)N;
-    radix_sort_pairs(skey, idx, k1, v1, N, bits, rs, s);
-    int nc = g.nkeys;
-    hipLaunchKernelGGL(k_fill_i32, dim3((nc + 255) / 256), dim3(256), 0, s, cstart, 0, nc);
-    hipLaunchKernelGGL(k_fill_i32, dim3((nc + 255) / 256), dim3(256), 0, s, cend, 0, nc);
-    hipLaunchKernelGGL(k_cell_ranges, dim3(nb), dim3(256), 0, s, skey, N, cstart, cend);
-    hipLaunchKernelGGL(k_gather_pos, dim3(nb), dim3(256), 0, s, x0, x1, x2, D, N, idx, pos, inv);
+    radix_sort_places(key, skey, idx, k1, v1, N, bits, rs, s);
+    hipLaunchKernelGGL(k_gather_pos, dim3(nb), dim3(256), 0, s, x0, x1, x2, D, N, skey, idx, pos, inv,
+                       cstart, cend);
 }
 
 void launch_pack_pos(const double *x0, const double *x1, const double *x2, int D, int N,
