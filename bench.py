@@ -38,7 +38,7 @@ VALU_ISSUE_PEAK = 256 * 2.4e9
 
 
 def face_kernel_bytes(D, tsz, k_mean):
-    """Algorithmic HBM bytes per particle of the faces+update kernel: own
+    """Algorithmic HBM bytes per particle of the faces+update stage: own
     position (double4), primitive record (8 values), face record (grads +
     B), FP64 state read (x, v, m, u), neighbour counts and row, next state
     written.  Neighbour records are gathered through the caches and not
@@ -90,8 +90,8 @@ def valu_roof(kernel, seconds):
 
 
 def roofline(kernel, seconds, bytes_per_launch, hbm_gbs):
-    """The dominant kernel's roofline.  The face kernel is bound by VALU
-    issue (its HBM traffic is a few % of peak): `achieved` / `peak` are VALU
+    """The dominant stage's roofline.  Where the committed PMC summary holds the
+    kernel's VALU count, it is priced by VALU issue: `achieved` / `peak` are VALU
     wave instructions per second (instructions per launch from the
     committed PMC summary, launch time from this run's HIP events), and the
     HBM figures (algorithmic bytes per launch over the same time, against
@@ -686,7 +686,9 @@ def main():
         head = dict(rate=learned[0], tim=learned[1], diag=learned[2], err=field_err(learned[3]),
                     drift=drift(learned[4]), seed="learned", train=learned[5])
 
-    face_kernel = "k_faces<3, float, %s>" % ("true" if head["seed"] == "learned" else "false")
+    # the face stage: two kernels (and the faces that wait for the learned seed)
+    face_kernel = "k_face_pairs<3, float, %s, 48> + k_face_sum<3, float>" % (
+        "true" if head["seed"] == "learned" else "false")
     k_mean = (d64["faces_solved"] / max(1, (W + K) * N))
     tface = float(head["tim"][3]) * 1e-3
     bytes_face = face_kernel_bytes(3, 4, k_mean) * N

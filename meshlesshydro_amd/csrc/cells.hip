@@ -4,18 +4,19 @@
 // createGhostParticles (:2113-2191), gridNNS (:324-365) and ghostNNS
 // (:2237-2260):
 //   1. cell key per particle with the reference's floor((x-min)/cellSize)
-//      (clamped when it equals the cell count), positions packed as double4;
-//   2. stable LSD radix sort of (cell key, particle index), 8-bit digits:
-//      LDS histogram per 2048-key tile, exclusive scan of the tile
+//      (clamped when it equals the cell count);
+//   2. stable LSD radix sort of (cell key, particle index), digits of up to
+//      9 bits: LDS histogram per 2048-key tile, exclusive scan of the tile
 //      histograms, then a scatter that ranks equal digits inside each
-//      wavefront with eight __ballot masks (match + popcount below the
+//      wavefront with one __ballot mask per bit (match + popcount below the
 //      lane), and across the block's waves through LDS counts;
 //   3. per-cell [start, end) ranges of the sorted order (ascending particle
-//      index inside a cell, as the reference's push_back lists);
+//      index inside a cell, as the reference's push_back lists); a small
+//      problem has 1 to 4 done by one block (k_cells_small);
 //   4. positions gathered into cell order as double4 (x, y, z, original
 //      index); cell keys follow a Morton curve (device_common.h), so that a
 //      block of the cell order is a compact brick of cells;
-//   5. one thread per particle, in work order: the 3^D stencil of
+//   5. one thread per particle (images: eight), in work order: the 3^D stencil of
 //      non-periodic cells (x outer ... z inner, Domain.cpp:83-118) with the
 //      strict test d^2 < h^2 in the reference's operation order, then the
 //      periodic images: every candidate in the window of virtual cells
