@@ -761,7 +761,8 @@ __device__ inline void search_one(const NbrArgs &a, int t, const Src &src, uint3
     const bool images = !err && has_images<D>(a, cc);
     a.nog[t] = images ? -1 : 0;
     segs[2] = (uint16_t)nb;
-    own_out = images ? 0 : (a.all_own ? cnt : (cnt > nb ? cnt - nb : 0));
+    // an overflowed row has no faces: its step keeps the state
+    own_out = images || err ? 0 : (a.all_own ? cnt : cnt - nb);
     if constexpr (kDens != 0) {
         // compDensity (Particles.cpp:1151-1184): the self term after the
         // real neighbours, then the images in ghost order (:2262-2290), which

@@ -1233,9 +1233,10 @@ __attribute__((amdgpu_waves_per_eu(MLH_FACES_WAVES(D, T, LEARNED)))) void k_face
     const bool live = t < a.N;
     FaceStats fs{};
     const int N = a.N;
-    if (a.flux && *a.nfaces <= a.fcap) return;  // k_face_pairs and k_face_sum did it all
+    const bool overflow = a.status[0] & kStatusErrMask;
+    if (a.flux && (overflow || *a.nfaces <= a.fcap)) return;  // k_face_sum did it all
     const int i = live ? (a.sidx ? (int)a.sidx[t] : t) : 0;
-    if (a.status[0] & kStatusErrMask) {
+    if (overflow) {
         // this step's neighbour search overflowed (the reference exits in
         // gridNNS / ghostNNS): the state is carried over unchanged
         if (live) particle_keep<D>(a, i);
@@ -1708,12 +1709,15 @@ __global__ __launch_bounds__(256) void k_face_sum(HydroArgs a) {
     constexpr int NF = D + 2, P = 256 / kSumLanes, U = 2, B = U * kSumLanes;
     __shared__ T s_flux[P][B][NF];
     __shared__ double s_sum[P][NF];
-    if (*a.nfaces > a.fcap) return;
+    // an overflowed search's slot count says nothing: whatever it is, the state
+    // is carried over below
+    const bool overflow = a.status[0] & kStatusErrMask;
+    if (!overflow && *a.nfaces > a.fcap) return;
     const int b0 = xcd_block() * P, N = a.N;
     const int p = (int)(threadIdx.x / kSumLanes), l = (int)(threadIdx.x & (kSumLanes - 1));
     const int t = b0 + p;
     if (a.deferred && b0 == 0 && threadIdx.x == 0) a.deferred[0].x = 0;  // for the next step
-    if (!(a.status[0] & kStatusErrMask)) {
+    if (!overflow) {
         const bool live = t < N;
         const int cnt = live ? a.noi[t] + a.nog[t] : 0;
         const uint32_t kt = live ? a.ck[t] : 0u;
@@ -1774,7 +1778,7 @@ __global__ __launch_bounds__(256) void k_face_sum(HydroArgs a) {
     const int u = b0 + (int)threadIdx.x;
     const bool live = u < N;
     const int i = live ? (a.sidx ? (int)a.sidx[u] : u) : 0;
-    if (a.status[0] & kStatusErrMask) {
+    if (overflow) {
         if (live) particle_keep<D>(a, i);
         return;
     }
