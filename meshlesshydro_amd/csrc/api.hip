@@ -56,6 +56,7 @@ struct mlh_ctx {
     void *flux = nullptr;
     unsigned long long flux_cap = 0;
     bool flux_fits = false;
+    bool pairs = false;  // whether this problem's faces are evaluated once at all
     uint16_t *face_rec = nullptr;
     uint2 *deferred = nullptr;  // (re)allocated with flux
     unsigned long long *nfaces = nullptr;
@@ -193,8 +194,15 @@ static int make_geom(mlh_ctx *c, const double *lo, const double *hi) {
     return 0;
 }
 
-// Slots for the faces' fluxes.  Without memory for them (or with rows too
-// long for the records) every face is evaluated from both sides.
+// Whether a problem's faces are evaluated once per pair: rows too long for the
+// records are not.  A matter of the parameters alone: the order of an FP32
+// learned step's sums follows it.
+static bool pairs_wanted(const mlh_params &p) {
+    return p.max_interactions <= kFaceRecMaxRow && p.max_ghost_interactions <= kFaceRecMaxRow;
+}
+
+// Slots for the faces' fluxes.  Without memory for them every face is
+// evaluated from both sides.
 constexpr size_t kFluxSmall = 64u << 20;   // bytes: given for the longest lists
 constexpr int kFluxPerParticle = 40;       // else at first: half of 72
                                            // neighbours, and some images
@@ -227,7 +235,7 @@ static void set_flux_slots(mlh_ctx *c, unsigned long long cap) {
 }
 static void first_flux_slots(mlh_ctx *c) {
     const mlh_params &p = c->p;
-    if (p.max_interactions > kFaceRecMaxRow || p.max_ghost_interactions > kFaceRecMaxRow) return;
+    if (!c->pairs) return;
     // a real pair has one slot, an image entry its own
     const unsigned long long N = c->N, D2 = c->D + 2;
     const unsigned long long rows = p.enforce_flux_sym ? (N * p.max_interactions + 1) / 2
@@ -277,6 +285,7 @@ static HydroArgs hydro_args(mlh_ctx *c) {
     a.nfaces = c->nfaces;
     a.fcap = c->flux_cap;
     a.flux_fits = c->flux_fits ? 1 : 0;
+    a.pairs = c->pairs ? 1 : 0;
     a.maxr = p.max_interactions;
     a.ck = co ? c->cell_key : c->sorted_key;
     for (int k = 0; k < 3; ++k) {
@@ -322,6 +331,7 @@ int mlh_create(const mlh_params *p, int32_t n, mlh_ctx **out) {
     c->prec = p->precision;
     c->tsz = c->prec == MLH_FP64 ? 8 : 4;
     c->stride = p->max_interactions + p->max_ghost_interactions;
+    c->pairs = pairs_wanted(*p);
     int st = p->periodic ? make_geom(c, p->box_min, p->box_max) : MLH_OK;
     if (st) { delete c; return st; }
     if (hipStreamCreateWithFlags(&c->s, hipStreamNonBlocking) != hipSuccess) {

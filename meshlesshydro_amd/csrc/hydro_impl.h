@@ -1214,20 +1214,24 @@ __device__ inline void add_counters(const HydroArgs &a, const FaceStats fs, int 
 #define MLH_FACES_WAVES(D, T, LEARNED) ((LEARNED && sizeof(T) == 4) ? 2 : 1)
 #endif
 
-// Faces of particle i, every one of its row evaluated here, where the fluxes
-// of k_face_pairs have no room.  LEARNED: the loop runs to the wavefront's largest
+// Faces of particle i, every one of its row evaluated here: the steps whose
+// fluxes have no room in k_face_pairs' slots, and the problems that take no slots
+// (HydroArgs::pairs).  LEARNED, in the loop: it runs to the wavefront's largest
 // neighbour count so that every lane takes part in the BF16 MFMA inference
 // of the p* seed for the wavefront's 64 faces of that iteration.
-template <int D, typename T, bool LEARNED>
+// FP32 learned: DEFER leaves the faces whose probe fails to the end of the row, and
+// adds them there.  In place of k_face_pairs they are seeded in the loop
+// instead, whose sums are then in row order as k_face_sum's: a step's bits do not
+// depend on whether its lists had room.  128^3 blast 2.78 ms deferred, 3.41 in
+// the loop; turbulence 160^3 12.9 and 23.6.
+template <int D, typename T, bool LEARNED, bool DEFER = false>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(MLH_FACES_WAVES(D, T, LEARNED)))) void k_faces(HydroArgs a) {
     constexpr int NF = D + 2;
     constexpr bool kFp32 = sizeof(T) == 4;
-    // FP32 learned: faces whose probe fails are deferred to the end of the
-    // row and seeded there by the network; the FP64 learned kernel runs the
-    // network inside the face loop, over the wavefront's longest row
-    constexpr bool kInLoopNet = LEARNED && !kFp32;
-    constexpr bool kDefer = LEARNED && kFp32;
+    constexpr bool kDefer = LEARNED && DEFER;
+    constexpr bool kInLoopNet = LEARNED && !kDefer;
+    static_assert(!DEFER || kFp32, "FP64 has no probe to defer by");
     __shared__ uint16_t lds[LEARNED ? 4 : 1][LEARNED ? 64 * 16 : 1];
     const int t = xcd_block() * blockDim.x + threadIdx.x;
     const bool live = t < a.N;
@@ -1282,12 +1286,13 @@ __attribute__((amdgpu_waves_per_eu(MLH_FACES_WAVES(D, T, LEARNED)))) void k_face
         const int it0 = fs.st.iters;
         if (act) face_of_entry<D, T>(a, t, i, e, jo, dt, fp, mp, self_lo, fs, kOwnView ? &own : nullptr);
         float seed = -1.f;
+        const bool far = LEARNED && kFp32 && act && mp.valid && !mp.accepted && mp.chg > kSeedGate;
         if constexpr (kInLoopNet) {
-            const bool strong = act && strong_jump<D, T>(a, fp);
-            if (__ballot(strong)) seed = face_net_seed<D, T>(a, strong, fp, lds[threadIdx.x >> 6], fs);
+            const bool net = kFp32 ? far : act && strong_jump<D, T>(a, fp);
+            if (__ballot(net)) seed = face_net_seed<D, T>(a, net, fp, lds[threadIdx.x >> 6], fs);
         }
         if (act) {
-            if (kDefer && mp.valid && !mp.accepted && mp.chg > kSeedGate) {
+            if (kDefer && far) {
                 // the standard guess was far off: Newton from the network's
                 // seed, after the row.  Entries 0..127 are marked in
                 // registers; for later ones (rows longer than 128) a flag
@@ -1299,7 +1304,9 @@ __attribute__((amdgpu_waves_per_eu(MLH_FACES_WAVES(D, T, LEARNED)))) void k_face
                 else defer_far = true;
                 for (int ax = 0; ax < D; ++ax) fp.A[ax] = T(0);
             }
-            face_accumulate<D, T>(a, fp, mp, seed, self_lo, it0, collect, acc, fs);
+            // a far face's probe does not count as one of its iterations
+            face_accumulate<D, T>(a, fp, mp, seed, self_lo, kInLoopNet && far ? fs.st.iters : it0,
+                                  collect, acc, fs);
         }
     }
     if constexpr (kDefer) {
@@ -1840,6 +1847,11 @@ __global__ __launch_bounds__(256) void k_sums(HydroArgs a, double *out) {
 template <int D, typename T, bool LEARNED>
 static void launch_faces_as(const HydroArgs &a, hipStream_t s) {
     const dim3 blk(256), rows((a.N + 255) / 256);
+    if constexpr (LEARNED && sizeof(T) == 4)
+        if (!a.pairs) {
+            hipLaunchKernelGGL((k_faces<D, T, true, true>), rows, blk, 0, s, a);
+            return;
+        }
     if (a.flux) {
         constexpr int G = kPairGroup<D, T>;
         HydroArgs p = a;
