@@ -194,11 +194,20 @@ static int make_geom(mlh_ctx *c, const double *lo, const double *hi) {
     return 0;
 }
 
-// Whether a problem's faces are evaluated once per pair: rows too long for the
-// records are not.  A matter of the parameters alone: the order of an FP32
-// learned step's sums follows it.
-static bool pairs_wanted(const mlh_params &p) {
-    return p.max_interactions <= kFaceRecMaxRow && p.max_ghost_interactions <= kFaceRecMaxRow;
+// Whether a problem's faces go through k_face_pairs and k_face_sum: rows too
+// long for the records do not.  Without flux symmetry the two sides of a face
+// differ and nothing is shared; there the pairs only deal a small problem's faces to
+// more wavefronts, and to fewer registers in 2D FP64.  Face stage without
+// symmetry, pairs against k_faces in us: 3D FP64 24^3 227 / 471, 40^3 506 / 496,
+// 56^3 1410 / 1183, 128^3 14260 / 11820; 3D FP32 24^3 94 / 294, 40^3 260 / 302, 56^3
+// 392 / 378, 128^3 3370 / 2690; 2D FP32 200^2 197 / 305, 350^2 404 / 360, 500^2
+// 662 / 651, 1000^2 2213 / 2302; 2D FP64 200^2 325 / 522, 1000^2 4052 / 4529.
+// A matter of the parameters and the size alone: the order of an FP32 learned
+// step's sums follows it.
+constexpr int kPairsNoSym = 1 << 16;
+static bool pairs_wanted(const mlh_params &p, int n) {
+    if (p.max_interactions > kFaceRecMaxRow || p.max_ghost_interactions > kFaceRecMaxRow) return false;
+    return p.enforce_flux_sym || n <= kPairsNoSym || (p.dim == 2 && p.precision == MLH_FP64);
 }
 
 // Slots for the faces' fluxes.  Without memory for them every face is
@@ -331,7 +340,7 @@ int mlh_create(const mlh_params *p, int32_t n, mlh_ctx **out) {
     c->prec = p->precision;
     c->tsz = c->prec == MLH_FP64 ? 8 : 4;
     c->stride = p->max_interactions + p->max_ghost_interactions;
-    c->pairs = pairs_wanted(*p);
+    c->pairs = pairs_wanted(*p, n);
     int st = p->periodic ? make_geom(c, p->box_min, p->box_max) : MLH_OK;
     if (st) { delete c; return st; }
     if (hipStreamCreateWithFlags(&c->s, hipStreamNonBlocking) != hipSuccess) {
