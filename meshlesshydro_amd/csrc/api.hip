@@ -56,6 +56,8 @@ struct mlh_ctx {
     void *flux = nullptr;
     unsigned long long flux_cap = 0;
     bool flux_fits = false;
+    unsigned long long flux_all = 0;         // slots the longest lists take
+    unsigned long long flux_refused = ~0ull; // too many since the last upload
     bool pairs = false;  // whether this problem's faces are evaluated once at all
     uint16_t *face_rec = nullptr;
     uint2 *deferred = nullptr;  // (re)allocated with flux
@@ -124,11 +126,29 @@ const char *mlh_last_error(void) { return g_last_error.c_str(); }
 
 }  // extern "C"
 
+static void drop_flux_slots(mlh_ctx *c) {
+    if (c->flux) hipFree(c->flux);  // waits for the device
+    if (c->deferred) hipFree(c->deferred);
+    c->flux = nullptr;
+    c->deferred = nullptr;
+    c->flux_cap = 0;
+    c->flux_fits = false;
+}
+
+// hipMalloc for a call of context c (null: none): where it is refused, again
+// once the context has given its face slots back, which it can do without
+hipError_t ctx_malloc(mlh_ctx *c, void **p, size_t bytes) {
+    const hipError_t e = hipMalloc(p, bytes ? bytes : 16);
+    if (e == hipSuccess || !c || !c->flux) return e;
+    hipGetLastError();
+    drop_flux_slots(c);
+    return hipMalloc(p, bytes ? bytes : 16);
+}
+
 template <typename P>
 static int dalloc(mlh_ctx *c, P **ptr, size_t bytes) {
     void *q = nullptr;
-    if (bytes == 0) bytes = 16;
-    hipError_t e = hipMalloc(&q, bytes);
+    hipError_t e = ctx_malloc(c, &q, bytes);
     if (e != hipSuccess)
         return fail(MLH_ERR_DEVICE, std::string("hipMalloc: ") + hipGetErrorString(e));
     c->allocs.push_back(q);
@@ -215,32 +235,45 @@ static bool pairs_wanted(const mlh_params &p, int n) {
 constexpr size_t kFluxSmall = 64u << 20;   // bytes: given for the longest lists
 constexpr int kFluxPerParticle = 40;       // else at first: half of 72
                                            // neighbours, and some images
-static void set_flux_slots(mlh_ctx *c, unsigned long long cap) {
-    const size_t bytes = (size_t)(c->D + 2) * c->tsz;
-    if (cap > 0xfffffff0ull) cap = 0xfffffff0ull;
-    void *q = nullptr;
-    uint2 *d = nullptr;
+// They take at most this part of the device memory that is free without
+// them: the rest is left to the caller's later allocations.
+constexpr int kFluxShare = 4;
+
+// Up to `want` slots in place of those there are, unless there would be fewer
+// than `need`.  What the old ones hold is lost, and given back first.
+static void set_flux_slots(mlh_ctx *c, unsigned long long want, unsigned long long need) {
+    const size_t slot = (size_t)(c->D + 2) * c->tsz;
+    const bool defer = c->prec == MLH_FP32 && c->p.riemann_seed == MLH_SEED_LEARNED;
     // FP32 learned: the list of rounds with deferred faces: 64 faces each but
     // the last two of a group (of four particles at least)
-    if (c->prec == MLH_FP32 && c->p.riemann_seed == MLH_SEED_LEARNED) {
-        const size_t n = 1 + (size_t)cap / 64 + 2 * ((size_t)c->N / 4 + 1);
-        if (hipMalloc((void **)&d, sizeof(uint2) * n) != hipSuccess ||
-            hipMemsetAsync(d, 0, sizeof(uint2), c->s) != hipSuccess) {
-            if (d) hipFree(d);
-            hipGetLastError();
-            return;  // as it was
-        }
-    }
-    if (hipMalloc(&q, bytes * cap) != hipSuccess) {
-        if (d) hipFree(d);
+    auto rounds = [&](unsigned long long cap) { return 1 + (size_t)cap / 64 + 2 * ((size_t)c->N / 4 + 1); };
+    size_t free = 0, total = 0;
+    if (hipMemGetInfo(&free, &total) != hipSuccess) {
         hipGetLastError();
         return;
     }
-    if (c->flux) hipFree(c->flux);
-    if (c->deferred) hipFree(c->deferred);
-    c->flux = q;
-    c->deferred = d;
-    c->flux_cap = cap;
+    const unsigned long long most = (free + c->flux_cap * slot) / kFluxShare / slot;
+    unsigned long long cap = want < most ? want : most;
+    if (cap > 0xfffffff0ull) cap = 0xfffffff0ull;
+    if (cap < need || cap <= c->flux_cap) {
+        c->flux_refused = need;
+        return;
+    }
+    const unsigned long long old = c->flux_cap;
+    drop_flux_slots(c);
+    for (unsigned long long n : {cap, old}) {
+        if (n == 0) break;
+        if (hipMalloc(&c->flux, slot * n) == hipSuccess &&
+            (!defer || (hipMalloc((void **)&c->deferred, sizeof(uint2) * rounds(n)) == hipSuccess &&
+                        hipMemsetAsync(c->deferred, 0, sizeof(uint2), c->s) == hipSuccess))) {
+            c->flux_cap = n;
+            c->flux_fits = n >= c->flux_all;
+            return;
+        }
+        hipGetLastError();
+        drop_flux_slots(c);
+        c->flux_refused = need;
+    }
 }
 static void first_flux_slots(mlh_ctx *c) {
     const mlh_params &p = c->p;
@@ -249,17 +282,16 @@ static void first_flux_slots(mlh_ctx *c) {
     const unsigned long long N = c->N, D2 = c->D + 2;
     const unsigned long long rows = p.enforce_flux_sym ? (N * p.max_interactions + 1) / 2
                                                        : N * p.max_interactions;
-    const unsigned long long all = rows + N * (p.periodic ? p.max_ghost_interactions : 0);
-    c->flux_fits = all * D2 * c->tsz <= kFluxSmall;
+    c->flux_all = rows + N * (p.periodic ? p.max_ghost_interactions : 0);
+    const bool small = c->flux_all * D2 * c->tsz <= kFluxSmall;
     const unsigned long long some = N * kFluxPerParticle * (p.enforce_flux_sym ? 1 : 2);
-    set_flux_slots(c, c->flux_fits || all < some ? all : some);
-    c->flux_fits = c->flux != nullptr && c->flux_cap >= all;
+    set_flux_slots(c, small || c->flux_all < some ? c->flux_all : some, 1);
 }
 // after a call whose faces did not fit (they were evaluated from both sides):
 // room for them and a quarter more
 static void grow_flux_slots(mlh_ctx *c, unsigned long long nfaces) {
-    if (c->flux && nfaces > c->flux_cap && c->flux_cap < 0xfffffff0ull)
-        set_flux_slots(c, nfaces + nfaces / 4);
+    if (c->flux && nfaces > c->flux_cap && nfaces < c->flux_refused)
+        set_flux_slots(c, nfaces + nfaces / 4, nfaces);
 }
 
 static HydroArgs hydro_args(mlh_ctx *c) {
@@ -431,8 +463,7 @@ int mlh_destroy(mlh_ctx *c) {
     mlp_free(c->mlp);
     for (hipEvent_t e : c->evpool) hipEventDestroy(e);
     if (c->dt_hist) hipFree(c->dt_hist);
-    if (c->flux) hipFree(c->flux);
-    if (c->deferred) hipFree(c->deferred);
+    drop_flux_slots(c);
     if (c->s_img) hipStreamSynchronize(c->s_img);
     if (c->ev_fork) hipEventDestroy(c->ev_fork);
     if (c->ev_join) hipEventDestroy(c->ev_join);
@@ -457,6 +488,7 @@ int mlh_upload_state(mlh_ctx *c, const double *x, const double *y, const double 
     HIPCHK(hipMemcpyAsync(c->u, u, b, hipMemcpyHostToDevice, c->s));
     HIPCHK(hipStreamSynchronize(c->s));
     c->stage = 0;
+    c->flux_refused = ~0ull;
     if (c->p.work_order == MLH_ORDER_AUTO) c->order = 0;  // settled at the next search
     return MLH_OK;
 }
@@ -505,8 +537,8 @@ static int prepare_open_grid(mlh_ctx *c) {
         if (c->cstart) hipFree(c->cstart);
         if (c->cend) hipFree(c->cend);
         c->cstart = c->cend = nullptr;
-        HIPCHK(hipMalloc(&c->cstart, 4 * (size_t)c->g.nkeys));
-        HIPCHK(hipMalloc(&c->cend, 4 * (size_t)c->g.nkeys));
+        HIPCHK(ctx_malloc(c, (void **)&c->cstart, 4 * (size_t)c->g.nkeys));
+        HIPCHK(ctx_malloc(c, (void **)&c->cend, 4 * (size_t)c->g.nkeys));
         c->cell_cap = c->g.nkeys;
     }
     return MLH_OK;
@@ -713,7 +745,7 @@ int mlh_run(mlh_ctx *c, int32_t n_steps, double dt_fixed, const double *dts_in,
     if (c->dt_hist_cap < n_steps) {
         if (c->dt_hist) hipFree(c->dt_hist);
         c->dt_hist = nullptr;
-        HIPCHK(hipMalloc(&c->dt_hist, sizeof(double) * 2 * (size_t)(n_steps > 0 ? n_steps : 1)));
+        HIPCHK(ctx_malloc(c, (void **)&c->dt_hist, sizeof(double) * 2 * (size_t)(n_steps > 0 ? n_steps : 1)));
         c->dt_hist_cap = n_steps;
     }
     double *dev_in = nullptr;
@@ -1128,8 +1160,8 @@ int mlh_riemann_flux_batch(mlh_ctx *c, int64_t n, const double *w_left, const do
     const size_t D = c->D, nw = (size_t)n * (D + 2), nv = (size_t)n * D;
     double *buf = nullptr;
     int *fl = nullptr;
-    HIPCHK(hipMalloc(&buf, sizeof(double) * (3 * nw + 2 * nv)));
-    if (hipMalloc(&fl, sizeof(int) * (size_t)n) != hipSuccess) {
+    HIPCHK(ctx_malloc(c, (void **)&buf, sizeof(double) * (3 * nw + 2 * nv)));
+    if (ctx_malloc(c, (void **)&fl, sizeof(int) * (size_t)n) != hipSuccess) {
         hipFree(buf);
         return fail(MLH_ERR_DEVICE, "hipMalloc failed");
     }
@@ -1162,7 +1194,7 @@ int mlh_set_face_collection(mlh_ctx *c, int64_t cap, int32_t particle_stride) {
     m.collect_stripes = 0;
     m.collect_stride = 0;
     if (particle_stride <= 0 || cap == 0) return MLH_OK;
-    HIPCHK(hipMalloc(&m.collect, sizeof(double) * 6 * (size_t)cap));
+    HIPCHK(ctx_malloc(c, (void **)&m.collect, sizeof(double) * 6 * (size_t)cap));
     // as many stripes as fit (a power of two, at most kCollectStripes), each
     // of cap / stripes rows; the rows past stripes * scap stay unused
     int stripes = 1;

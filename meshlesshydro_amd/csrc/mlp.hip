@@ -755,8 +755,8 @@ __global__ __launch_bounds__(256) void k_epoch_keys(uint32_t *__restrict__ key,
     } while (0)
 
 template <typename P>
-static hipError_t dmalloc(P **p, size_t bytes) {
-    return hipMalloc((void **)p, bytes ? bytes : 16);
+static hipError_t dmalloc(mlh_ctx *c, P **p, size_t bytes) {
+    return ctx_malloc(c, (void **)p, bytes);
 }
 
 // device buffer freed at scope exit
@@ -771,11 +771,11 @@ struct DevBuf {
 static int ensure_mlp(mlh_ctx *c) {
     MlpState &m = ctx_mlp(c);
     if (!m.params) {
-        CHK(dmalloc(&m.params, sizeof(float) * kMlpN));
-        CHK(dmalloc(&m.frags, sizeof(MlpFrags)));
-        CHK(dmalloc(&m.adam_m, sizeof(float) * kMlpN));
-        CHK(dmalloc(&m.adam_v, sizeof(float) * kMlpN));
-        CHK(dmalloc(&m.grad, sizeof(float) * kMlpN));
+        CHK(dmalloc(c, &m.params, sizeof(float) * kMlpN));
+        CHK(dmalloc(c, &m.frags, sizeof(MlpFrags)));
+        CHK(dmalloc(c, &m.adam_m, sizeof(float) * kMlpN));
+        CHK(dmalloc(c, &m.adam_v, sizeof(float) * kMlpN));
+        CHK(dmalloc(c, &m.grad, sizeof(float) * kMlpN));
         CHK(hipMemset(m.adam_m, 0, sizeof(float) * kMlpN));
         CHK(hipMemset(m.adam_v, 0, sizeof(float) * kMlpN));
         m.adam_t = 0;
@@ -845,16 +845,16 @@ struct TrainBufs {
 static int train_chunks(int batch) { return (batch + kTrainChunk - 1) / kTrainChunk; }
 
 // n samples; partial sums for batches of up to max_batch samples
-static int alloc_train(TrainBufs &b, int64_t n, int max_batch) {
-    CHK(dmalloc(&b.X, sizeof(float) * n * kMlpIn));
-    CHK(dmalloc(&b.T, sizeof(float) * n));
-    CHK(dmalloc(&b.partial, sizeof(float) * (size_t)train_chunks(max_batch) * kPartialN));
-    CHK(dmalloc(&b.loss, sizeof(float)));
-    CHK(dmalloc(&b.idx, sizeof(int) * n));
-    CHK(dmalloc(&b.pk, sizeof(uint32_t) * n));
-    CHK(dmalloc(&b.pk1, sizeof(uint32_t) * n));
-    CHK(dmalloc(&b.pv1, sizeof(uint32_t) * n));
-    CHK(dmalloc(&b.scr, sizeof(uint32_t) * radix_sort_scratch_words((int)n)));
+static int alloc_train(mlh_ctx *c, TrainBufs &b, int64_t n, int max_batch) {
+    CHK(dmalloc(c, &b.X, sizeof(float) * n * kMlpIn));
+    CHK(dmalloc(c, &b.T, sizeof(float) * n));
+    CHK(dmalloc(c, &b.partial, sizeof(float) * (size_t)train_chunks(max_batch) * kPartialN));
+    CHK(dmalloc(c, &b.loss, sizeof(float)));
+    CHK(dmalloc(c, &b.idx, sizeof(int) * n));
+    CHK(dmalloc(c, &b.pk, sizeof(uint32_t) * n));
+    CHK(dmalloc(c, &b.pk1, sizeof(uint32_t) * n));
+    CHK(dmalloc(c, &b.pv1, sizeof(uint32_t) * n));
+    CHK(dmalloc(c, &b.scr, sizeof(uint32_t) * radix_sort_scratch_words((int)n)));
     return MLH_OK;
 }
 
@@ -921,15 +921,15 @@ static int build_set(mlh_ctx *c, const double *F6, const unsigned long long *cou
     DevBuf<uint8_t> cls;
     DevBuf<unsigned long long> cnt;  // trivial, non-trivial, kept
     DevBuf<unsigned long long> blk;  // per-block counts
-    CHK(dmalloc(&Xall.p, sizeof(float) * kMlpIn * nslots));
-    CHK(dmalloc(&Tall.p, sizeof(float) * nslots));
+    CHK(dmalloc(c, &Xall.p, sizeof(float) * kMlpIn * nslots));
+    CHK(dmalloc(c, &Tall.p, sizeof(float) * nslots));
     uint32_t **u[] = {&hlo.p, &hhi.p, &khi.p, &ord.p, &k1.p, &v1.p};
-    for (uint32_t **q : u) CHK(dmalloc(q, sizeof(uint32_t) * nslots));
-    CHK(dmalloc(&scr.p, sizeof(uint32_t) * radix_sort_scratch_words((int)nslots)));
-    CHK(dmalloc(&cls.p, nslots));
+    for (uint32_t **q : u) CHK(dmalloc(c, q, sizeof(uint32_t) * nslots));
+    CHK(dmalloc(c, &scr.p, sizeof(uint32_t) * radix_sort_scratch_words((int)nslots)));
+    CHK(dmalloc(c, &cls.p, nslots));
     const int64_t nb = (nslots + 255) / 256;
-    CHK(dmalloc(&cnt.p, sizeof(unsigned long long) * 3));
-    CHK(dmalloc(&blk.p, sizeof(unsigned long long) * 2 * nb));
+    CHK(dmalloc(c, &cnt.p, sizeof(unsigned long long) * 3));
+    CHK(dmalloc(c, &blk.p, sizeof(unsigned long long) * 2 * nb));
     hipLaunchKernelGGL(k_ds_prep, dim3(nb), dim3(256), 0, s, F6, counts, scap, nslots, gamma,
                        Xall.p, Tall.p, hlo.p, hhi.p, cls.p, blk.p);
     hipLaunchKernelGGL(k_sum_u64, dim3(1), dim3(256), 0, s, blk.p, (int)nb, cnt.p);
@@ -969,7 +969,7 @@ static int build_set(mlh_ctx *c, const double *F6, const unsigned long long *cou
     CHK(hipMemcpyAsync(h + 2, cnt.p + 2, sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
     CHK(hipStreamSynchronize(s));
     dc.nsel = (int64_t)h[2];
-    int st = alloc_train(b, dc.nsel, max_batch > 65536 ? max_batch : 65536);
+    int st = alloc_train(c, b, dc.nsel, max_batch > 65536 ? max_batch : 65536);
     if (st) return st;
     if (dc.nsel > 0)
         hipLaunchKernelGGL(k_ds_gather, dim3((dc.nsel + 255) / 256), dim3(256), 0, s, ord.p,
@@ -1010,7 +1010,7 @@ static int train_on_set(mlh_ctx *c, TrainBufs &b, const DsCounts &dc, int n_epoc
     int st = train_epochs(c, b, nval, ntrain, n_epochs, batch, lr, seed, &last);
     if (st) return st;
     DevBuf<float> Y;
-    CHK(dmalloc(&Y.p, sizeof(float) * nval));
+    CHK(dmalloc(c, &Y.p, sizeof(float) * nval));
     hipLaunchKernelGGL(k_mlp_infer_bf16, dim3((nval + 255) / 256), dim3(256), 0, s, m.frags, b.X,
                        nval, Y.p);
     std::vector<float> y(nval), t(nval);
@@ -1040,7 +1040,7 @@ int mlh_mlp_loss_grad(mlh_ctx *c, int64_t n, const float *feats, const float *ta
     MlpState &m = ctx_mlp(c);
     if (!m.params) return ctx_fail(MLH_ERR_NOT_TRAINED, "no network parameters");
     TrainBufs b;
-    int st = alloc_train(b, n, (int)n);
+    int st = alloc_train(c, b, n, (int)n);
     if (st) return st;
     hipStream_t s = ctx_stream(c);
     CHK(hipMemcpyAsync(b.X, feats, sizeof(float) * n * kMlpIn, hipMemcpyHostToDevice, s));
@@ -1061,7 +1061,7 @@ int mlh_mlp_train(mlh_ctx *c, int64_t n, const float *feats, const float *target
     hipStream_t s = ctx_stream(c);
     if (batch > n) batch = (int)n;
     TrainBufs b;
-    if ((st = alloc_train(b, n, batch))) return st;
+    if ((st = alloc_train(c, b, n, batch))) return st;
     CHK(hipMemcpyAsync(b.X, feats, sizeof(float) * n * kMlpIn, hipMemcpyHostToDevice, s));
     CHK(hipMemcpyAsync(b.T, target, sizeof(float) * n, hipMemcpyHostToDevice, s));
     float last = 0.f;
@@ -1080,7 +1080,7 @@ int mlh_mlp_train_faces(mlh_ctx *c, int64_t n, const double *states6, double gam
     if (!m.params) return ctx_fail(MLH_ERR_NOT_TRAINED, "no network parameters to train from");
     hipStream_t s = ctx_stream(c);
     DevBuf<double> F6;
-    CHK(dmalloc(&F6.p, sizeof(double) * 6 * n));
+    CHK(dmalloc(c, &F6.p, sizeof(double) * 6 * n));
     CHK(hipMemcpyAsync(F6.p, states6, sizeof(double) * 6 * n, hipMemcpyHostToDevice, s));
     TrainBufs b;
     DsCounts dc;
@@ -1124,7 +1124,7 @@ int mlh_mlp_dataset(mlh_ctx *c, int64_t n, const double *states6, double gamma,
     const unsigned long long *counts = nullptr;
     int64_t scap = n, nslots = n;
     if (states6) {
-        CHK(dmalloc(&F6.p, sizeof(double) * 6 * n));
+        CHK(dmalloc(c, &F6.p, sizeof(double) * 6 * n));
         CHK(hipMemcpyAsync(F6.p, states6, sizeof(double) * 6 * n, hipMemcpyHostToDevice, s));
         src = F6.p;
     } else {
@@ -1178,8 +1178,8 @@ int mlh_mlp_infer(mlh_ctx *c, int64_t n, const float *feats, float *out, int32_t
     if (!m.params) return ctx_fail(MLH_ERR_NOT_TRAINED, "no network parameters");
     hipStream_t s = ctx_stream(c);
     float *X = nullptr, *Y = nullptr;
-    CHK(dmalloc(&X, sizeof(float) * n * kMlpIn));
-    CHK(dmalloc(&Y, sizeof(float) * n));
+    CHK(dmalloc(c, &X, sizeof(float) * n * kMlpIn));
+    CHK(dmalloc(c, &Y, sizeof(float) * n));
     hipMemcpyAsync(X, feats, sizeof(float) * n * kMlpIn, hipMemcpyHostToDevice, s);
     int64_t nb = (n + 255) / 256;
     if (bf16)
@@ -1213,9 +1213,9 @@ int mlh_riemann_exact_batch(mlh_ctx *c, int64_t n, double gamma, const double *r
     double *buf = nullptr;
     int *ib = nullptr;
     unsigned long long *fb = nullptr;
-    CHK(dmalloc(&buf, sizeof(double) * n * 9));
-    CHK(dmalloc(&ib, sizeof(int) * n * 2));
-    CHK(dmalloc(&fb, sizeof(unsigned long long)));
+    CHK(dmalloc(c, &buf, sizeof(double) * n * 9));
+    CHK(dmalloc(c, &ib, sizeof(int) * n * 2));
+    CHK(dmalloc(c, &fb, sizeof(unsigned long long)));
     size_t b = sizeof(double) * n;
     const double *in[6] = {rhoL, uL, PL, rhoR, uR, PR};
     for (int k = 0; k < 6; ++k) hipMemcpyAsync(buf + k * n, in[k], b, hipMemcpyHostToDevice, s);
@@ -1277,7 +1277,7 @@ int mlh_riemann_exact_batch_device(mlh_ctx *c, int64_t n, double gamma, const do
     if (n == 0) return MLH_OK;
     hipStream_t s = c ? ctx_stream(c) : nullptr;
     unsigned long long *fb = nullptr;
-    CHK(dmalloc(&fb, sizeof(unsigned long long)));
+    CHK(dmalloc(c, &fb, sizeof(unsigned long long)));
     hipEvent_t e0, e1;
     hipEventCreate(&e0);
     hipEventCreate(&e1);
@@ -1379,9 +1379,9 @@ int mlh_riemann_pstar_batch(int64_t n, double gamma, const double *rhoL, const d
     double *buf = nullptr;
     int *ib = nullptr;
     unsigned long long *fb = nullptr;
-    CHK(dmalloc(&buf, sizeof(double) * n * 7));
-    CHK(dmalloc(&ib, sizeof(int) * n));
-    CHK(dmalloc(&fb, sizeof(unsigned long long)));
+    CHK(dmalloc(nullptr, &buf, sizeof(double) * n * 7));
+    CHK(dmalloc(nullptr, &ib, sizeof(int) * n));
+    CHK(dmalloc(nullptr, &fb, sizeof(unsigned long long)));
     size_t b = sizeof(double) * n;
     const double *in[6] = {rhoL, uL, PL, rhoR, uR, PR};
     for (int k = 0; k < 6; ++k) hipMemcpy(buf + k * n, in[k], b, hipMemcpyHostToDevice);

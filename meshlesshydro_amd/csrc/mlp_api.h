@@ -46,3 +46,5 @@ mlh::MlpState &ctx_mlp(mlh_ctx *c);
 hipStream_t ctx_stream(mlh_ctx *c);
 double ctx_gamma(mlh_ctx *c);  // the context's adiabatic index
 int ctx_fail(int code, const char *msg);
+// hipMalloc, at the cost of the context's face slots where there is no room
+hipError_t ctx_malloc(mlh_ctx *c, void **p, size_t bytes);

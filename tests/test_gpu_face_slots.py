@@ -3,6 +3,7 @@ and what is left of the device."""
 import ctypes as C
 import gc
 
+import numpy as np
 import pytest
 
 from cases import jitter3d, relerr
@@ -50,3 +51,70 @@ def test_no_flux_symmetry_vs_oracle(n, hip, oracle_mod):
     sim.close()
     for k in gs:
         assert relerr(gs[k], os_[k]) < 1e-9, k
+
+
+class Fill:
+    """All but `leave` bytes of the free device memory, while in scope."""
+
+    def __init__(self, hip, leave):
+        self.hip = hip
+        n = free_bytes(hip) - leave
+        assert n > 0
+        self.buf = hip.DeviceBuffer(n, np.uint8)
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        self.buf.free()
+
+
+def used_by(hip, p, s):
+    """(device memory of a context for state s, free memory with it)"""
+    before = free_bytes(hip)
+    sim = hip.Simulation(p, s)
+    after = free_bytes(hip)
+    sim.close()
+    return before - after, after
+
+
+def test_slots_leave_the_device_to_others(hip):
+    """Slots take a quarter at most of what is free without them."""
+    p, s = jitter3d(100, debug_level=0)
+    gc.collect()
+    with Fill(hip, 6 << 30):
+        with_slots, free = used_by(hip, p, s)
+        p.enforce_flux_sym = 0
+        without, _ = used_by(hip, p, s)
+        slots = with_slots - without
+        print(f"\n[slots] {slots >> 20} MiB of {(free + slots) >> 20}", flush=True)
+        # 40 slots of 40 bytes a particle would be 1526 MiB
+        assert 0 < slots <= (free + slots) // 4 + (64 << 20)
+
+
+def test_slots_make_room_for_the_face_arrays(hip):
+    """A stage whose arrays the slots leave no room for gets the slots' memory,
+    and the context goes on without them: the same bits."""
+    p, s = jitter3d(100, debug_level=0, max_interactions=96, max_ghost_interactions=64)
+    arrays = s["x"].size * (96 + 64) * 8 * 21
+    slots = s["x"].size * 40 * 40
+    ref = hip.Simulation(p, s)
+    sim = hip.Simulation(p, s)
+    with Fill(hip, arrays - 3 * slots // 4):
+        out = []
+        for q in (ref, sim):
+            q.neighbours()
+            q.density()
+            dt = q.timestep()
+            q.gradients()
+            if q is sim:
+                q.effective_faces()
+            q.upload(s)
+            q.run(2)
+            out.append((dt, q.state()))
+        sim.close()
+    ref.close()
+    (dt0, s0), (dt1, s1) = out
+    assert dt0 == dt1
+    for k in s0:
+        assert np.array_equal(s0[k], s1[k]), k
