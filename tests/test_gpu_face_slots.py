@@ -118,3 +118,23 @@ def test_slots_make_room_for_the_face_arrays(hip):
     assert dt0 == dt1
     for k in s0:
         assert np.array_equal(s0[k], s1[k]), k
+
+
+def test_long_rows_have_slots_from_the_second_step(hip):
+    """Rows of 125 entries outgrow the slots a context starts with: only the first
+    step of a fresh context's run evaluates its faces from both sides (1.4 times
+    the face stage of the pairs), so the run is within 1.2 of a second one."""
+    p, s = jitter3d(56, kernel_size=3.1 / 56, debug_level=0, max_interactions=200, max_ghost_interactions=200)
+    sim = hip.Simulation(p, s)
+    ms, out = [], []
+    for k in range(2):
+        print(f"\n[long rows] run {k}", flush=True)
+        sim.upload(s)
+        dts = sim.run(8)
+        ms.append(float(sim.timings()[3]))
+        out.append((dts, sim.state()))
+    sim.close()
+    assert ms[0] < 1.2 * ms[1], ms
+    assert np.array_equal(out[0][0], out[1][0])
+    for k in out[0][1]:
+        assert np.array_equal(out[0][1][k], out[1][1][k]), k
