@@ -1155,6 +1155,11 @@ __global__ void k_pack_pos(const double *__restrict__ x0, const double *__restri
 // block does all of it: 10^4 particles 38 us against 85 in 16 launches, 1024
 // particles 10 us against 32 and the gaps between 11.
 constexpr int kSmallKeys = 1 << 16;
+// Threads of k_assign_cells at least, while there are as many cells: the chip's, so
+// that a sparse cloud's few particles do not clear its many cells alone (10^4
+// particles in 10^7 cells: 64 us with a thread each, 20 so; 2 x 10^4 in 1.25 x 10^8:
+// 227 and 185; the search of 600 in 10^7: 978 and 234).
+constexpr int kClearThreads = 256 * 2048;
 void launch_cells(const Geom &g, int D, const double *x0, const double *x1,
                   const double *x2, int N, double4 *pos, uint32_t *key, uint32_t *idx,
                   uint32_t *skey, uint32_t *scratch, int *cstart, int *cend, uint32_t *inv,
@@ -1172,11 +1177,13 @@ void launch_cells(const Geom &g, int D, const double *x0, const double *x1,
                                passes, dbits, key, idx, skey, cstart, cend, pos, inv, nfaces);
         return;
     }
+    const int clear = ((g.nkeys < kClearThreads ? g.nkeys : kClearThreads) + 255) / 256;
+    const dim3 assign(nb > clear ? nb : clear);
     if (D == 2)
-        hipLaunchKernelGGL(k_assign_cells<2>, dim3(nb), dim3(256), 0, s, g, x0, x1, x2, N, key, cstart,
+        hipLaunchKernelGGL(k_assign_cells<2>, assign, dim3(256), 0, s, g, x0, x1, x2, N, key, cstart,
                            cend, nfaces);
     else
-        hipLaunchKernelGGL(k_assign_cells<3>, dim3(nb), dim3(256), 0, s, g, x0, x1, x2, N, key, cstart,
+        hipLaunchKernelGGL(k_assign_cells<3>, assign, dim3(256), 0, s, g, x0, x1, x2, N, key, cstart,
                            cend, nfaces);
     uint32_t *k1 = scratch, *v1 = scratch + N, *rs = scratch + 2 * (size_t)N;
     radix_sort_places(key, skey, idx, k1, v1, N, bits, rs, s);
