@@ -56,6 +56,8 @@ struct mlh_ctx {
     void *flux = nullptr;
     unsigned long long flux_cap = 0;
     bool flux_fits = false;
+    bool flux_full = false;                  // slots for flux_limit or the longest lists
+    unsigned long long flux_limit = 0;       // most slots a step makes use of
     unsigned long long flux_all = 0;         // slots the longest lists take
     unsigned long long flux_refused = ~0ull; // too many since the last upload
     unsigned long long last_faces = ~0ull;   // slots the last call took, ~0: none since
@@ -133,7 +135,7 @@ static void drop_flux_slots(mlh_ctx *c) {
     c->flux = nullptr;
     c->deferred = nullptr;
     c->flux_cap = 0;
-    c->flux_fits = false;
+    c->flux_fits = c->flux_full = false;
 }
 
 // hipMalloc for a call of context c (null: none): where it is refused, again
@@ -231,6 +233,25 @@ static bool pairs_wanted(const mlh_params &p, int n) {
     return p.enforce_flux_sym || n <= kPairsNoSym || (p.dim == 2 && p.precision == MLH_FP64);
 }
 
+// Slots beyond which a step's faces are evaluated from both sides although they
+// could be stored: k_face_sum looks a mirrored entry up in its partner's row, at
+// a cost that grows with the row, the evaluation it saves does not.  Entries a
+// row at which both take the same time: FP64 2D 550, 3D 600, learned seed (which
+// runs the network for every evaluation) past 700; FP32 2D 260, 3D 150 to 270.
+// Face stage in ms, both sides against pairs: 48^3 turbulence, 374 entries FP64
+// 6.21 / 5.02, FP32 2.37 / 2.85, 683 entries 11.15 / 10.33 and 4.18 / 6.37; 700^2
+// FP32 163 entries 4.14 / 3.41, 366 entries 8.72 / 10.37.  Few particles leave
+// k_faces too few wavefronts: there the line lies higher (FP32 24^3 683 entries 3.18
+// / 1.28, 32^3 374 1.83 / 1.20, 40^3 259 1.32 / 1.21, 374 1.88 / 1.97, learned 3.59
+// / 2.00; 200^2 367 entries 2.03 / 1.70, 652 3.15 / 3.87).
+static unsigned long long pairs_limit(const mlh_params &p, int n) {
+    if (!p.enforce_flux_sym) return ~0ull;  // nothing to look up
+    const bool fp64 = p.precision == MLH_FP64, net = p.riemann_seed == MLH_SEED_LEARNED;
+    const int each = fp64 ? (net ? 400 : 256) : (p.dim == 2 ? 130 : 100);
+    const int few = fp64 || p.dim == 2 ? 1 << 16 : net ? 1 << 18 : 1 << 17;
+    return (unsigned long long)each * (n > few ? n : few);
+}
+
 // Slots for the faces' fluxes.  Without memory for them every face is
 // evaluated from both sides.
 constexpr size_t kFluxSmall = 64u << 20;   // bytes: given for the longest lists
@@ -255,6 +276,7 @@ static void set_flux_slots(mlh_ctx *c, unsigned long long want, unsigned long lo
     }
     const unsigned long long most = (free + c->flux_cap * slot) / kFluxShare / slot;
     unsigned long long cap = want < most ? want : most;
+    if (cap > c->flux_limit) cap = c->flux_limit;
     if (cap > 0xfffffff0ull) cap = 0xfffffff0ull;
     if (cap < need || cap <= c->flux_cap) {
         c->flux_refused = need;
@@ -269,6 +291,7 @@ static void set_flux_slots(mlh_ctx *c, unsigned long long want, unsigned long lo
                         hipMemsetAsync(c->deferred, 0, sizeof(uint2), c->s) == hipSuccess))) {
             c->flux_cap = n;
             c->flux_fits = n >= c->flux_all;
+            c->flux_full = c->flux_fits || n >= c->flux_limit;
             return;
         }
         hipGetLastError();
@@ -284,6 +307,7 @@ static void first_flux_slots(mlh_ctx *c) {
     const unsigned long long rows = p.enforce_flux_sym ? (N * p.max_interactions + 1) / 2
                                                        : N * p.max_interactions;
     c->flux_all = rows + N * (p.periodic ? p.max_ghost_interactions : 0);
+    c->flux_limit = pairs_limit(p, c->N);
     const bool small = c->flux_all * D2 * c->tsz <= kFluxSmall;
     const unsigned long long some = N * kFluxPerParticle * (p.enforce_flux_sym ? 1 : 2);
     set_flux_slots(c, small || c->flux_all < some ? c->flux_all : some, 1);
@@ -291,7 +315,7 @@ static void first_flux_slots(mlh_ctx *c) {
 // where faces did not fit (they were evaluated from both sides): room for them
 // and a quarter more
 static void grow_flux_slots(mlh_ctx *c, unsigned long long nfaces) {
-    if (c->flux && nfaces > c->flux_cap && nfaces < c->flux_refused)
+    if (c->flux && nfaces > c->flux_cap && nfaces <= c->flux_limit && nfaces < c->flux_refused)
         set_flux_slots(c, nfaces + nfaces / 4, nfaces);
 }
 
@@ -327,6 +351,9 @@ static HydroArgs hydro_args(mlh_ctx *c) {
     a.nfaces = c->nfaces;
     a.fcap = c->flux_cap;
     a.flux_fits = c->flux_fits ? 1 : 0;
+    a.flux_full = c->flux_full ? 1 : 0;
+    a.flimit = c->flux_limit;
+    a.always_pairs = c->flux_all <= c->flux_limit ? 1 : 0;
     a.pairs = c->pairs ? 1 : 0;
     a.maxr = p.max_interactions;
     a.ck = co ? c->cell_key : c->sorted_key;
@@ -646,7 +673,8 @@ static int check_status(mlh_ctx *c) {
 // entries a row, face stage of a fresh context's six steps: 7.70 ms a step without
 // this, 5.77 with it (5.50 in a second run).
 static int fit_flux_slots(mlh_ctx *c, hipEvent_t searched) {
-    if (!c->flux || c->flux_fits || c->last_faces <= c->flux_cap) return MLH_OK;
+    // (calls since the upload have had their slots)
+    if (!c->flux || c->flux_full || c->last_faces != ~0ull) return MLH_OK;
     HIPCHK(hipEventSynchronize(searched));
     unsigned long long n = 0;
     HIPCHK(hipMemcpy(&n, c->nfaces, sizeof(n), hipMemcpyDeviceToHost));

@@ -1220,9 +1220,9 @@ __device__ inline void add_counters(const HydroArgs &a, const FaceStats fs, int 
 // neighbour count so that every lane takes part in the BF16 MFMA inference
 // of the p* seed for the wavefront's 64 faces of that iteration.
 // FP32 learned: DEFER leaves the faces whose probe fails to the end of the row, and
-// adds them there.  In place of k_face_pairs they are seeded in the loop
-// instead, whose sums are then in row order as k_face_sum's: a step's bits do not
-// depend on whether its lists had room.  128^3 blast 2.78 ms deferred, 3.41 in
+// adds them there.  In place of k_face_pairs (up to a.flimit faces) they are
+// seeded in the loop instead, whose sums are then in row order as k_face_sum's: a
+// step's bits do not depend on whether its lists had room.  128^3 blast 2.78 ms deferred, 3.41 in
 // the loop; turbulence 160^3 12.9 and 23.6.
 template <int D, typename T, bool LEARNED, bool DEFER = false>
 __global__ __launch_bounds__(256)
@@ -1239,6 +1239,8 @@ __attribute__((amdgpu_waves_per_eu(MLH_FACES_WAVES(D, T, LEARNED)))) void k_face
     const int N = a.N;
     const bool overflow = a.status[0] & kStatusErrMask;
     if (a.flux && (overflow || *a.nfaces <= a.fcap)) return;  // k_face_sum did it all
+    if (LEARNED && kFp32 && a.pairs && (overflow ? DEFER : (*a.nfaces > a.flimit) != DEFER))
+        return;  // the other instantiation's step
     const int i = live ? (a.sidx ? (int)a.sidx[t] : t) : 0;
     if (overflow) {
         // this step's neighbour search overflowed (the reference exits in
@@ -1847,11 +1849,11 @@ __global__ __launch_bounds__(256) void k_sums(HydroArgs a, double *out) {
 template <int D, typename T, bool LEARNED>
 static void launch_faces_as(const HydroArgs &a, hipStream_t s) {
     const dim3 blk(256), rows((a.N + 255) / 256);
-    if constexpr (LEARNED && sizeof(T) == 4)
-        if (!a.pairs) {
+    if constexpr (LEARNED && sizeof(T) == 4) {
+        if (!a.pairs || !a.always_pairs)
             hipLaunchKernelGGL((k_faces<D, T, true, true>), rows, blk, 0, s, a);
-            return;
-        }
+        if (!a.pairs) return;
+    }
     if (a.flux) {
         constexpr int G = kPairGroup<D, T>;
         HydroArgs p = a;
@@ -1863,7 +1865,7 @@ static void launch_faces_as(const HydroArgs &a, hipStream_t s) {
             hipLaunchKernelGGL((k_face_deferred<D, G>), dim3(kDeferredBlocks), dim3(64), 0, s, p);
         hipLaunchKernelGGL((k_face_sum<D, T>), dim3((a.N + 256 / kSumLanes - 1) / (256 / kSumLanes)),
                            blk, 0, s, a);
-        if (a.flux_fits) return;
+        if (a.flux_fits || (LEARNED && sizeof(T) == 4 && a.flux_full)) return;
     }
     hipLaunchKernelGGL((k_faces<D, T, LEARNED>), rows, blk, 0, s, a);
 }

@@ -64,13 +64,16 @@ struct HydroArgs {
     // [fcap][D+2] of T, null when every face is evaluated from both sides;
     // *nfaces > fcap: they do not fit, and the step evaluates both sides;
     // flux_fits: they fit whatever the neighbour lists are
-    // pairs: this problem's faces are evaluated once wherever they fit
+    // pairs: this problem's faces are evaluated once wherever they fit, up to
+    // flimit of them (always_pairs: whatever the lists are; flux_full: there is
+    // room for as many)
     void *flux;
     const uint16_t *face_rec;
     const unsigned long long *nfaces;
     unsigned long long fcap;
-    int flux_fits;
-    int pairs;
+    int flux_fits, flux_full;
+    int pairs, always_pairs;
+    unsigned long long flimit;
     int face_group;              // particles per wavefront of k_face_pairs
     uint2 *deferred;             // FP32 learned: rounds with deferred faces
     int maxr;

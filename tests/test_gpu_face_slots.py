@@ -7,7 +7,8 @@ import numpy as np
 import pytest
 
 from cases import jitter3d, relerr
-from meshlesshydro_amd._abi import MLH_FP32, MLH_FP64
+from meshlesshydro_amd import learned as L
+from meshlesshydro_amd._abi import MLH_FP32, MLH_FP64, MLH_SEED_LEARNED
 
 pytestmark = pytest.mark.gpu
 
@@ -138,3 +139,27 @@ def test_long_rows_have_slots_from_the_second_step(hip):
     assert np.array_equal(out[0][0], out[1][0])
     for k in out[0][1]:
         assert np.array_equal(out[0][1][k], out[1][1][k]), k
+
+
+@pytest.mark.parametrize("seed", ["standard", "learned"])
+def test_very_long_rows_are_no_slower_in_pairs(seed, hip):
+    """Rows of 600 entries, where looking a mirrored entry up costs more than the
+    evaluation it saves (1.5 times the face stage): the faces are evaluated
+    from both sides, as without flux symmetry."""
+    p, s = jitter3d(48, kernel_size=5.24 / 48, debug_level=0, max_interactions=1000, max_ghost_interactions=1000,
+                    precision=MLH_FP32)
+    if seed == "learned":
+        p.riemann_seed = MLH_SEED_LEARNED
+    ms = []
+    for sym in (1, 0):
+        p.enforce_flux_sym = sym
+        sim = hip.Simulation(p, s)
+        if seed == "learned":
+            sim.mlp_set_params(L.init_params(1))
+        for k in range(3):
+            print(f"\n[very long rows {seed}] symmetry {sym} run {k}", flush=True)
+            sim.upload(s)
+            sim.run(2)
+        ms.append(float(sim.timings()[3]))
+        sim.close()
+    assert ms[0] < 1.2 * ms[1], ms
