@@ -296,7 +296,7 @@ void radix_sort_pairs(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, in
 // here holds a contiguous sixteenth of the particles in registers and moves them
 // through LDS once per digit.
 constexpr int kSmallThreads = 1024, kSmallWaves = kSmallThreads / 64;
-constexpr int kSmallRounds = 16;
+constexpr int kSmallRounds = 10;
 constexpr int kSmallCells = kSmallThreads * kSmallRounds;  // most particles
 template <int D>
 __global__ __launch_bounds__(kSmallThreads) void k_cells_small(
@@ -1151,10 +1151,14 @@ __global__ void k_pack_pos(const double *__restrict__ x0, const double *__restri
     pos[i] = make_double4(x0[i], x1[i], D == 3 ? x2[i] : 0.0, (double)i);
 }
 
-// Up to kSmallCells particles and kSmallKeys cells (which k_cells_small clears) one
-// block does all of it: 10^4 particles 38 us against 85 in 16 launches, 1024
-// particles 10 us against 32 and the gaps between 11.
-constexpr int kSmallKeys = 1 << 16;
+// A small problem's list is one block's work as long as that is shorter than the
+// other way's launches: kSmallCells particles, 32 cells to clear counted as one,
+// kSmallKeys cells.
+// Search group of a step in us, one block against launches: 10^4 lattice particles
+// 112 / 131, 10^4 random ones on 32^2 cells 123 / 127, on 128^2 89 / 91, on 250^2
+// 96 / 87 (past the line), on 32^3 124 / 111 (past it); 8000 on 250^2 86 / 81, on
+// 32^3 113 / 110; 14000 on 64^2 122 / 100; 1000 on 32^2 53 / 82.
+constexpr int kSmallKeysPer = 32, kSmallKeys = 1 << 16;
 // Threads of k_assign_cells at least, while there are as many cells: the chip's, so
 // that a sparse cloud's few particles do not clear its many cells alone (10^4
 // particles in 10^7 cells: 64 us with a thread each, 20 so; 2 x 10^4 in 1.25 x 10^8:
@@ -1167,7 +1171,7 @@ void launch_cells(const Geom &g, int D, const double *x0, const double *x1,
     int nb = (N + 255) / 256;
     int bits = 1;
     while ((1 << bits) < g.nkeys) ++bits;
-    if (N <= kSmallCells && g.nkeys <= kSmallKeys) {
+    if (N + g.nkeys / kSmallKeysPer <= kSmallCells && g.nkeys <= kSmallKeys) {
         const int passes = (bits + kRsMaxBits - 1) / kRsMaxBits, dbits = (bits + passes - 1) / passes;
         if (D == 2)
             hipLaunchKernelGGL(k_cells_small<2>, dim3(1), dim3(kSmallThreads), 0, s, g, x0, x1, x2, N,
