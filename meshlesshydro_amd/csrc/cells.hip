@@ -548,12 +548,12 @@ __device__ inline bool is_image(const Geom &g, const int *s, const double4 &pj, 
 //    stage as sort words (parent << 6 | (7 - axis mask) << 3 | shift signs:
 //    ascending words are the ghost order, see stage_word), each placed by a
 //    binary search; they go to the row as work positions (a.inv) when the
-//    search ends.  Parents from 2^26 on skip the stage.
+//    search ends.  Problems of more than 2^26 particles have no stage.
 //  * Further hits (more images than the stage holds) are insertion-sorted
 //    in the row itself, each key read back through the entry's position.
 template <int D, bool kCaller>
 __device__ inline int image_search(const NbrArgs &a, int t, const double *xi, const int *cc,
-                                   int g0, uint32_t *stage, int ss) {
+                                   int g0, uint32_t *stage) {
     const Geom &g = a.g;
     const int N = a.N;
     int gcnt = 0, err = 0;
@@ -592,25 +592,25 @@ __device__ inline int image_search(const NbrArgs &a, int t, const double *xi, co
                             int lo = 0, hi = gcnt;
                             while (lo < hi) {
                                 const int mid = (lo + hi) >> 1;
-                                if (stage[mid * ss] <= w) lo = mid + 1;
+                                if (stage[mid] <= w) lo = mid + 1;
                                 else hi = mid;
                             }
                             int p = gcnt;
                             for (; p - 4 >= lo; p -= 4) {
                                 uint32_t b[4];
 #pragma unroll
-                                for (int u = 0; u < 4; ++u) b[u] = stage[(p - 1 - u) * ss];
+                                for (int u = 0; u < 4; ++u) b[u] = stage[p - 1 - u];
 #pragma unroll
-                                for (int u = 0; u < 4; ++u) stage[(p - u) * ss] = b[u];
+                                for (int u = 0; u < 4; ++u) stage[p - u] = b[u];
                             }
-                            for (; p > lo; --p) stage[p * ss] = stage[(p - 1) * ss];
-                            stage[p * ss] = w;
+                            for (; p > lo; --p) stage[p] = stage[p - 1];
+                            stage[p] = w;
                             ++gcnt;
                             return;
                         }
                         const uint64_t ke = ghost_key(jo, code);
                         if (!in_row) {
-                            for (int k = 0; k < gcnt; ++k) nb[nb_slot(N, t, g0 + k)] = to_row(stage[k * ss]);
+                            for (int k = 0; k < gcnt; ++k) nb[nb_slot(N, t, g0 + k)] = to_row(stage[k]);
                             in_row = true;
                         }
                         int p = gcnt;
@@ -637,7 +637,7 @@ __device__ inline int image_search(const NbrArgs &a, int t, const double *xi, co
                     }
                 }
         if (!in_row)
-            for (int k = 0; k < gcnt; ++k) nb[nb_slot(N, t, g0 + k)] = to_row(stage[k * ss]);
+            for (int k = 0; k < gcnt; ++k) nb[nb_slot(N, t, g0 + k)] = to_row(stage[k]);
         if (err) atomicOr(a.status, 1 << 3);
     }
     return gcnt;
@@ -826,8 +826,8 @@ __device__ inline uint32_t face_slots(unsigned long long *nfaces, int own) {
 // eight at a time, kImgLanes lanes to a particle: each lane takes every eighth
 // cell of the window and appends its hits to the particle's LDS stage in any
 // order; the sort words are distinct, so a hit's place in the row is the number
-// of smaller words.  A particle whose images do not fit the stage, the capacity
-// or the words goes through image_search on one lane.
+// of smaller words.  A particle whose images do not fit the stage or the capacity
+// goes through image_search on one lane.
 // A wavefront's time is its particles' dependent loads, not the work: one
 // particle per lane 97 us at 32^2, 594 at 24^3, 206 at 1000^2; here 27, 122, 167
 // (turbulence 160^3 with `per` 64 1391 -> 1041; blast 128^3 589 -> 663, beside
@@ -887,9 +887,9 @@ __global__ __launch_bounds__(kImgThreads) void k_images(NbrArgs a, int per) {
         wave_lds_sync();
         const int n = (int)s_n[grp];
         if (on) {
-            if (n > kGroupStage || n > a.maxg || (uint32_t)a.N > (1u << kStageIdxBits)) {
+            if (n > kGroupStage || n > a.maxg) {
                 if (l == 0)
-                    a.img_cnt[t] = image_search<D, kCaller>(a, t, xi, cc, a.img_base, s_stage[grp], 1);
+                    a.img_cnt[t] = image_search<D, kCaller>(a, t, xi, cc, a.img_base, s_stage[grp]);
             } else {
                 for (int e = l; e < n; e += kImgLanes) {
                     const uint32_t w = s_stage[grp][e];
@@ -902,6 +902,21 @@ __global__ __launch_bounds__(kImgThreads) void k_images(NbrArgs a, int per) {
         }
         wave_lds_sync();
     }
+}
+
+// The same with one particle per lane, sorted in its row: the problems whose
+// parents the sort words do not hold (8200^2, 56 neighbours: 1.85 ms; through
+// k_images, which would leave seven of eight lanes idle, 12.65).
+template <int D, bool kCaller>
+__global__ __launch_bounds__(kImgThreads) void k_images_rows(NbrArgs a) {
+    const int t = xcd_block() * blockDim.x + threadIdx.x;
+    if (t >= a.N) return;
+    int cc[3];
+    cell_coords<D>(a.g, a.ck_w[t], cc);
+    if (!has_images<D>(a, cc)) return;
+    const double4 pi = a.pos_w[t];
+    const double xi[3] = {pi.x, pi.y, pi.z};
+    a.img_cnt[t] = image_search<D, kCaller>(a, t, xi, cc, a.img_base, nullptr);
 }
 
 // After k_neighbours and k_images: for the particles k_neighbours left their
@@ -1218,8 +1233,11 @@ static void launch_nbr_dens(const NbrArgs &a, dim3 grid, const NbrStreams &st) {
         hipEventRecord(st.fork, st.s);
         hipStreamWaitEvent(st.s_img, st.fork, 0);
         const int per = a.N <= kImgSpread ? kImgGroups : kImgThreads;
-        hipLaunchKernelGGL((k_images<D, kCaller>), dim3((a.N + per - 1) / per), dim3(kImgThreads),
-                           0, st.s_img, a, per);
+        const dim3 images((a.N + per - 1) / per);
+        if ((uint32_t)a.N > (1u << kStageIdxBits))
+            hipLaunchKernelGGL((k_images_rows<D, kCaller>), images, dim3(kImgThreads), 0, st.s_img, a);
+        else
+            hipLaunchKernelGGL((k_images<D, kCaller>), images, dim3(kImgThreads), 0, st.s_img, a, per);
         hipEventRecord(st.join, st.s_img);
     }
     hipLaunchKernelGGL((k_neighbours<D, kCaller, kDens>), grid, dim3(256), 0, st.s, a);
