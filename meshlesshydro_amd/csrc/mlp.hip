@@ -534,8 +534,13 @@ __global__ __launch_bounds__(256) void k_riemann_few(const BatchArgs a) {
 // Solves a.n faces on s; the number of blocks.  At most kBatchBlocks (two to
 // three times what is resident at once): a wavefront's lists pay from a few rounds
 // on, and its last ones are part empty.  2^24 states FP64: 1024 blocks 2.33 ms,
-// 1536 2.22, 2048 2.23, 3072 2.34.
-constexpr int kBatchBlocks = 1536;
+// 1536 2.22, 2048 2.23, 3072 2.34.  Fewer faces give a wavefront of so many blocks
+// two to ten rounds, and the last blocks a turn of their own: below 2^22 two
+// thirds as many.  2^20 states, 1536 against 1024 blocks: random FP64 426 / 344
+// us, near-uniform 70 / 65, with the learned seed FP32 97 / 88; 2^21 near-uniform
+// 128 / 121 and 180 / 166.
+constexpr int kBatchBlocks = 1536, kBatchBlocksFew = 1024;
+constexpr int64_t kBatchMany = 1 << 22;
 // Up to kFewFaces each face in one go: there the lists' rounds come one after the
 // other with nothing beside them.  Random / near-uniform states FP64, in
 // one go against lists: 2^18 241 / 22 us against 275 / 23, 2^19 365 / 36 against
@@ -549,7 +554,8 @@ static int launch_riemann_as(BatchArgs a, hipStream_t s) {
         hipLaunchKernelGGL((k_riemann_few<MODE, LEARNED>), dim3(rounds), dim3(256), 0, s, a);
         return (int)rounds;
     }
-    a.tiles = (int)((rounds + kBatchBlocks - 1) / kBatchBlocks);
+    const int most = a.n < kBatchMany ? kBatchBlocksFew : kBatchBlocks;
+    a.tiles = (int)((rounds + most - 1) / most);
     const int blocks = (int)((rounds + a.tiles - 1) / a.tiles);
     hipLaunchKernelGGL((k_riemann_batch<MODE, LEARNED>), dim3(blocks), dim3(256), 0, s, a);
     return blocks;
