@@ -37,76 +37,87 @@ HBM_PEAK_GBS = 8000.0
 VALU_ISSUE_PEAK = 256 * 2.4e9
 
 
+# cycles of a vector-memory address unit
+ADDRESS_PEAK = 2.4e9
+
+
+def face_kernels(seed):
+    """Name of the FP32 face stage of the 3D step: its kernels."""
+    learned = seed == "learned"
+    names = ["k_face_pairs<3, float, %s, 48>" % ("true" if learned else "false"), "k_face_sum<3, float>"]
+    if learned:  # the faces that wait for the network's seed
+        names.insert(1, "k_face_deferred<3, 48>")
+    return " + ".join(names)
+
+
 def face_kernel_bytes(D, tsz, k_mean):
-    """Algorithmic HBM bytes per particle of the faces+update stage: own
-    position (double4), primitive record (8 values), face record (grads +
-    B), FP64 state read (x, v, m, u), neighbour counts and row, next state
-    written.  Neighbour records are gathered through the caches and not
-    counted."""
+    """Algorithmic HBM bytes per particle of the faces+update stage.
+    k_face_pairs: own position (double4), primitive record (8 values), face
+    record (grads + B), slot record and neighbour counts, its half of the row,
+    a flux written for every pair.  k_face_sum: counts and slot record, the
+    row, the flux of every entry, FP64 state read (x, v, m, u), next state
+    written.  Records gathered through the caches (the neighbours', and the
+    partners' rows that mirrored entries are looked up in) are not counted."""
     nf = D + 2
     frn = nf * D + D * D
-    own = 32 + 8 * tsz + frn * tsz + 8 * (2 * D + 2) + 8
-    row = 4 * k_mean
-    write = 8 * (2 * D + 2)
-    return own + row + write
+    slots = 2 * (8 if D == 2 else 16)
+    flux = nf * tsz
+    pairs = 32 + 8 * tsz + frn * tsz + slots + 8 + 0.5 * k_mean * (4 + flux)
+    sums = slots + 8 + k_mean * (4 + flux) + 2 * 8 * (2 * D + 2)
+    return pairs + sums
 
 
 def profiled(key, kernel):
     """A per-launch figure of `kernel` from the committed rocprofv3 PMC
     summary profiles/pmc_traffic_blast128.md: the line `<key> <kernel> =
-    <value>`, or None when absent.  Keys: traffic_bytes_per_launch (HBM
-    bytes, FETCH_SIZE + WRITE_SIZE each scaled by the counters of a 1 GiB
-    copy) and valu_instr_per_launch (SQ_INSTS_VALU, wave instructions)."""
+    <value>`, for a stage ("a + b") the sum of its kernels', or None when one
+    is absent.  Keys: traffic_bytes_per_launch (HBM bytes, FETCH_SIZE +
+    WRITE_SIZE each scaled by the counters of a 1 GiB copy),
+    valu_instr_per_launch (SQ_INSTS_VALU, wave instructions) and
+    ta_busy_cycles_per_launch (TA_BUSY_avr, busy cycles of the vector-memory
+    address units)."""
     path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles",
                         "pmc_traffic_blast128.md")
+    found = {}
     try:
         with open(path) as fh:
             for line in fh:
                 line = line.strip().strip("`")
                 if line.startswith(key + " ") and "=" in line:
                     name, val = line[len(key) + 1:].rsplit("=", 1)
-                    if name.strip() == kernel:
-                        return float(val)
+                    found[name.strip()] = float(val)
     except OSError:
         pass
-    return None
-
-
-def measured_traffic(kernel):
-    """HBM bytes per launch of `kernel` from the committed PMC summary."""
-    return profiled("traffic_bytes_per_launch", kernel)
-
-
-def valu_roof(kernel, seconds):
-    """The face kernel's VALU issue rate against the chip's: wave-level
-    VALU instructions per launch (committed PMC summary) over the launch
-    time measured in this run."""
-    instr = profiled("valu_instr_per_launch", kernel)
-    if instr is None or seconds <= 0:
-        return None
-    rate = instr / seconds
-    return {"instr_per_launch": instr, "achieved_per_s": rate, "peak_per_s": VALU_ISSUE_PEAK,
-            "frac": rate / VALU_ISSUE_PEAK}
+    names = kernel.split(" + ")
+    return sum(found[k] for k in names) if all(k in found for k in names) else None
 
 
 def roofline(kernel, seconds, bytes_per_launch, hbm_gbs):
-    """The dominant stage's roofline.  Where the committed PMC summary holds the
-    kernel's VALU count, it is priced by VALU issue: `achieved` / `peak` are VALU
-    wave instructions per second (instructions per launch from the
-    committed PMC summary, launch time from this run's HIP events), and the
-    HBM figures (algorithmic bytes per launch over the same time, against
-    8 TB/s) follow as a secondary roof."""
-    v = valu_roof(kernel, seconds)
+    """The dominant stage's roofline, by the unit it keeps busiest: VALU issue
+    (wave instructions per second) or vector-memory addressing (busy cycles
+    per second of an address unit), each per launch from the committed PMC
+    summary over the launch time of this run's HIP events.  The other follows as
+    a secondary roof, and so do the HBM figures (algorithmic bytes per launch
+    over the same time, against 8 TB/s).  For kernels the summary does not hold,
+    the bound is not known: HBM alone is priced."""
     hbm = {"achieved": hbm_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": hbm_gbs / HBM_PEAK_GBS,
            "algorithmic_bytes_per_launch": bytes_per_launch}
-    base = {"kernel": kernel, "traffic": measured_traffic(kernel), "launch_ms": 1e3 * seconds,
-            "hbm": hbm}
-    if v is None:  # no VALU count in the committed profile: HBM only
-        return dict(base, bound="hbm", achieved=hbm_gbs, peak=HBM_PEAK_GBS, unit="GB/s",
+    base = {"kernel": kernel, "traffic": profiled("traffic_bytes_per_launch", kernel),
+            "launch_ms": 1e3 * seconds, "hbm": hbm}
+    roofs = {}
+    for name, key, peak, unit in (
+            ("valu", "valu_instr_per_launch", VALU_ISSUE_PEAK, "VALU wave-instructions/s"),
+            ("vector_memory_addressing", "ta_busy_cycles_per_launch", ADDRESS_PEAK,
+             "busy cycles/s of an address unit")):
+        n = profiled(key, kernel)
+        if n is not None and seconds > 0:
+            roofs[name] = {"achieved": n / seconds, "peak": peak, "unit": unit, "frac": n / seconds / peak,
+                           key: n}
+    if not roofs:
+        return dict(base, bound="not measured", achieved=hbm_gbs, peak=HBM_PEAK_GBS, unit="GB/s",
                     frac=hbm_gbs / HBM_PEAK_GBS)
-    return dict(base, bound="valu", achieved=v["achieved_per_s"], peak=v["peak_per_s"],
-                unit="VALU wave-instructions/s", frac=v["frac"],
-                valu_instr_per_launch=v["instr_per_launch"])
+    bound = max(roofs, key=lambda k: roofs[k]["frac"])
+    return dict(base, bound=bound, **roofs.pop(bound), **roofs)
 
 
 def sedov_run(args, state, base, log):
@@ -686,9 +697,7 @@ def main():
         head = dict(rate=learned[0], tim=learned[1], diag=learned[2], err=field_err(learned[3]),
                     drift=drift(learned[4]), seed="learned", train=learned[5])
 
-    # the face stage: two kernels (and the faces that wait for the learned seed)
-    face_kernel = "k_face_pairs<3, float, %s, 48> + k_face_sum<3, float>" % (
-        "true" if head["seed"] == "learned" else "false")
+    face_kernel = face_kernels(head["seed"])
     k_mean = (d64["faces_solved"] / max(1, (W + K) * N))
     tface = float(head["tim"][3]) * 1e-3
     bytes_face = face_kernel_bytes(3, 4, k_mean) * N
