@@ -130,7 +130,9 @@ const char *mlh_last_error(void) { return g_last_error.c_str(); }
 }  // extern "C"
 
 static void drop_flux_slots(mlh_ctx *c) {
-    if (c->flux) hipFree(c->flux);  // waits for the device
+    // a run's steps may be under way with them
+    if (c->flux || c->deferred) hipStreamSynchronize(c->s);
+    if (c->flux) hipFree(c->flux);
     if (c->deferred) hipFree(c->deferred);
     c->flux = nullptr;
     c->deferred = nullptr;
