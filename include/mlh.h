@@ -142,7 +142,9 @@ typedef struct mlh_ctx mlh_ctx;
 void mlh_params_default(mlh_params *p);
 int mlh_version(void);
 /* Particles(int N) (Particles.cpp:67-149) + MeshlessScheme ctor
- * (MeshlessScheme.cpp:8-19): allocates device arrays for n particles. */
+ * (MeshlessScheme.cpp:8-19): allocates device arrays for n particles.  Beside
+ * them it takes room for the fluxes of the faces, at most a quarter of the
+ * memory that is then free, and gives it back where a later one of its own is refused. */
 int mlh_create(const mlh_params *p, int32_t n, mlh_ctx **out);
 int mlh_destroy(mlh_ctx *ctx);
 const char *mlh_last_error(void);

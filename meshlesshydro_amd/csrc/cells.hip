@@ -27,9 +27,8 @@
 //      away per axis, so the window is complete: the result equals the
 //      reference's exhaustive ghost loop.
 // Neighbour entries hold work positions (cell-order positions, or original
-// indices when the work order is the caller's); rows are stored transposed
-// (entry n of work position t at nbr[n*N + t]) so that the writes here and
-// the reads of the per-particle kernels are coalesced.  Inside one cell the
+// indices when the work order is the caller's); rows are stored in chunks of
+// eight entries (nb_slot), one 32-byte sector each.  Inside one cell the
 // cell order is ascending original index (stable sort of the identity), so
 // the reference's neighbour order is kept.
 #include <hip/hip_runtime.h>
@@ -477,11 +476,8 @@ __device__ inline bool has_images(const NbrArgs &a, const int *cc) {
     return near_edge;
 }
 
-// Entries a thread's image search sorts in its LDS stage before they go to
-// the row (more images than this continue with the row's own insertion).
-// 40 holds every image of the 3D lattice with h = 2.4 dx (5 to 40 per
-// particle, mean 12) and keeps the image kernel at four wavefronts per SIMD
-// (10 KB of LDS per wavefront).
+// Entries image_search sorts in its lane's LDS stage before they go to the row
+// (more images than this continue with the row's own insertion).
 constexpr int kImgStage = 40;
 // parents of staged images lie below 2^kStageIdxBits
 constexpr int kStageIdxBits = 26;
@@ -544,7 +540,7 @@ __device__ inline bool is_image(const Geom &g, const int *s, const double4 &pj, 
 // particles whose cell lies within the image window of a domain face
 // search.  Returns the image count (an overflow sets the status bit and
 // keeps the entries found so far).
-//  * The first kImgStage hits are insertion-sorted in the thread's LDS
+//  * The first kImgStage hits are insertion-sorted in the lane's LDS
 //    stage as sort words (parent << 6 | (7 - axis mask) << 3 | shift signs:
 //    ascending words are the ghost order, see stage_word), each placed by a
 //    binary search; they go to the row as work positions (a.inv) when the

@@ -25,8 +25,8 @@ void launch_gradients_fp32(const HydroArgs &a, int D, hipStream_t s) {
 }
 
 void launch_faces_fp32(const HydroArgs &a, int D, hipStream_t s) {
-    // learned: faces whose standard guess was far off are solved after the
-    // row from the network's seed, inside the same kernel
+    // learned: faces whose standard guess was far off are solved from the
+    // network's seed by k_face_deferred (without pairs: after the row, in k_faces)
     if (D == 2) launch_faces_of<2, float>(a, s);
     else launch_faces_of<3, float>(a, s);
 }

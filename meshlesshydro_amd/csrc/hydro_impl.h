@@ -1522,8 +1522,9 @@ constexpr uint32_t kDeferredTag = 0x7fc5eed1u;
 // One wavefront per block, face_group particles each: their views are held in
 // LDS, their faces dealt to the lanes as one list.  The records of a round's 64
 // neighbours go straight to LDS while the round before is being solved.
-// Bound by VALU issue (FP32) and by the latency of dependent FP64 operations at
-// one wavefront per SIMD (FP64, 304 registers; held to 256 it spills and takes
+// Bound in FP32 by latency at two wavefronts per SIMD (235 registers; VALU 0.59
+// busy, the address units 0.51), in FP64 by that of dependent operations at
+// one (304 registers; held to 256 it spills and takes
 // 8.4 ms instead of 7.3 at 128^3).  The list, not a row per lane, because own
 // faces per particle differ (11 to 45 on a lattice with 28 on average: a row
 // per lane took 2.20 ms in FP32, the list 1.74, with direct loads to LDS 1.45);
@@ -1706,8 +1707,8 @@ __device__ inline void mirror_row(const HydroArgs &a, int q, const MirrorPlace &
 // The flux sums of the particles from the stored faces, in row order (the
 // reference's collectFluxes order), and the update.  A mirrored entry takes
 // the partner's flux with the opposite sign, so F_ji = -F_ij bitwise.
-// Bound by the L1's cache accesses: the lookups take about 0.6 of its 1.27 ms
-// at 128^3 FP32, the fluxes 0.4, the state 0.25.  One thread per particle took
+// Bound by vector-memory addressing (address units 0.84 busy, VALU 0.31): the
+// lookups take about 0.6 of its 1.27 ms at 128^3 FP32, the fluxes 0.4, the state 0.25.  One thread per particle took
 // 2.4 ms: 64 rows of slots in flight per wavefront push each other out of L2.
 // Eight lanes per particle and sixteen entries at a time: each lane looks up
 // and loads the fluxes of two entries, then (through LDS) lane c sums

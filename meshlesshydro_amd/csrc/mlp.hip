@@ -328,10 +328,10 @@ __global__ __launch_bounds__(256) void k_mlp_infer_bf16(const MlpFrags *__restri
 // for a mean of 5.5.  So a solve stops after kCapFirst iterations (78% of
 // random states are done; FP32 mode: before any FP64 iteration) and what is
 // left waits on the wavefront's lists in LDS until 64 such faces can go on
-// together: list 0 up to kCapSecond, list 1 to the end.  FP64 issue bounds
-// it (80% of the time at three wavefronts per SIMD).
-// 2^24 random states FP64: 9.9 ms in one go, 2.2 ms; 2^26 FP32: standard seed
-// 41 -> 8.4 ms, learned seed 13.4 -> 7.5 ms.  Caps 4/11 to 6/12: 2.2 to 2.4 ms.
+// together: list 0 up to kCapSecond, list 1 to the end.  VALU issue bounds
+// it (0.85 busy in FP64 at 2.4 wavefronts per SIMD, 0.73 in FP32 at 1.7).
+// 2^24 random states FP64: 9.9 ms in one go, 2.0 ms; 2^26 FP32: standard seed
+// 41 -> 8.0 ms, learned seed 13.4 -> 7.1 ms.  Caps 4/11 to 6/12: 2.2 to 2.4 ms.
 // A list per block in place of one per wavefront: 2.2 ms FP64, 1.1 ms more
 // learned; the next states loaded ahead: 45 registers more, spilled.  Learned
 // seed: weights kept in registers 1 wavefront per SIMD, 14 ms; read for one
