@@ -58,16 +58,19 @@ class Fill:
     """All but `leave` bytes of the free device memory, while in scope."""
 
     def __init__(self, hip, leave):
-        self.hip = hip
+        self.bufs = []
         n = free_bytes(hip) - leave
         assert n > 0
-        self.buf = hip.DeviceBuffer(n, np.uint8)
+        while n > 0:
+            self.bufs.append(hip.DeviceBuffer(min(n, 16 << 30), np.uint8))
+            n -= 16 << 30
 
     def __enter__(self):
         return self
 
     def __exit__(self, *exc):
-        self.buf.free()
+        for b in self.bufs:
+            b.free()
 
 
 def used_by(hip, p, s):

@@ -60,7 +60,7 @@ def test_search_time(hip):
         print(f"\n[{n}^3 particles]", flush=True)
         sim = hip.Simulation(p, lattice(n, 3))
         t = []
-        for _ in range(4):
+        for _ in range(10):
             t0 = time.perf_counter()
             sim.neighbours()
             t.append(1e3 * (time.perf_counter() - t0))
